@@ -306,11 +306,11 @@ def work(case):
 def tolerance(case):
     # About four times the largest error against 64 bits seen over the listed
     # and some drawn cases: 2.5e-3 in bf16 and 3.1e-4 in fp16 (the rounding of
-    # the stored outputs and, in attention, of the weights as operands), 3.1e-7
+    # the stored outputs and, in attention, of the weights as operands), 4.5e-7
     # in fp32 (sums of up to thousands of terms).
     if case["kind"] == "pad":
         return "exact"
-    return {"rel": {"fp32": 1.3e-6, "fp16": 1.3e-3, "bf16": 1e-2}[case["dtype"]]}
+    return {"rel": {"fp32": 1.8e-6, "fp16": 1.3e-3, "bf16": 1e-2}[case["dtype"]]}
 
 
 # ------------------------------------------------------------------- exact
