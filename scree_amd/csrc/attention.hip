@@ -42,6 +42,7 @@ constexpr int kBN = 64;         // keys per staged block (forward, dQ)
 constexpr int kMaxBatch = 2048; // sequences the sorting scheduler handles (more: natural order)
 constexpr int kMaxClass = 4096; // row blocks per sequence it sorts (longer: natural order)
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kNegInf = -__builtin_inff();
 
 // ------------------------------------------------------------ workspace
@@ -1893,60 +1894,36 @@ __global__ __launch_bounds__(kThreads, (dkv_waves<D, CAUSAL>())) void attn_bwd_d
   }
 }
 
-// ---------------------------------------------------------- fp32 attention
-// fp32 inputs, which the reference's Array-level function computes as given
-// (its torch branch, reference/varlen_attention.py:90-113).  The matrix
-// instructions run fp32 at a sixteenth of their 16-bit rate, so these kernels
-// use FP32 FMAs instead: each row of an item (a query, or a key for dK/dV) is
-// split over TPR consecutive lanes holding DPT columns each (DPT = 16, or 4-8
-// for small launches, below), a dot product is DPT FMAs plus a DPP sum over
-// those lanes, and K / V (or Q / dO)
+// ------------------------------------------- fp32 attention at head_dim 256
+// The matrix-instruction kernels below hold up to head_dim 128 in registers;
+// at 256 these use FP32 FMAs: each row of an item (a query, or a key for
+// dK/dV) is split over TPR consecutive lanes holding 16 columns each, a dot
+// product is 16 FMAs plus a DPP sum over those lanes, and K / V (or Q / dO)
 // rows are staged 32 at a time in LDS, where every row group of a wave reads
 // the same staged row (a broadcast); the next 32 rows are loaded into
 // registers while the current ones are used.  Two workgroups share an item,
-// 64 rows each (in passes of 32 rows at head_dim 256), which doubles the
-// workgroups a small problem spreads over the CUs.  Scores, weights, sums and
-// accumulators are fp32; the forward takes each 32-key tile's maximum before
-// forming its weights, so every weight is at most 1, as in the reference's
-// max-subtracted softmax.  Every sum over keys or queries is taken per
-// 32-row tile first and then over the tiles, which keeps its rounding error
-// near that of the blocked sums of a GEMM (a group of 4 heads over 1,000
-// queries otherwise added 3x the reference's own fp32 error to dV).  Same
-// work lists, item order and failure handling as the 16-bit kernels.
+// 64 rows each in passes of 32 rows.  Scores, weights, sums and accumulators
+// are fp32; the forward takes each 32-key tile's maximum before forming its
+// weights, so every weight is at most 1, as in the reference's
+// max-subtracted softmax.  Every sum over keys or queries is taken per 32-row
+// tile first and then over the tiles, which keeps its rounding error near
+// that of the blocked sums of a GEMM.  Same work lists, item order and
+// failure handling as the 16-bit kernels.
 constexpr int kF32Split = 2;                // workgroups per item
 constexpr int kF32WgRows = kBM / kF32Split;  // rows of an item per workgroup
 constexpr int kF32Rows = 32;                // keys (forward, dQ) or queries (dK/dV) per LDS tile
-// Columns per lane: 16 (the narrow form), or, for launches too small to
-// give every SIMD a wave in that form, max(4, D / 16) (the wide form: 4 to
-// 16 lanes per row, so each row's chain of keys is 2-4x shorter and a
-// workgroup holds up to 4x the waves, at the price of repeating each row's
-// softmax arithmetic on more lanes).  Both keep every row within 16 lanes.
-// Measured (MI355X, causal): config 1's 1,980 tokens x 4 heads x 32, a
-// narrow grid of 512 waves, run 56 -> 30 us forward and 182 -> 100 us
-// forward + backward in the wide form (with its two key groups, below);
-// 7,168 tokens x 8 heads x 64 (3,776 narrow waves) ran 13 % (forward) and
-// 41 % (forward + backward) slower with the wider rows, so only launches
-// below one narrow wave per SIMD take them.
-constexpr int kF32NarrowDpt = 16;
+constexpr int kF32Dpt = 16;                 // columns per lane
 template <int D>
-constexpr int f32_wide_dpt() {
-  return D / 16 > 4 ? D / 16 : 4;
-}
-template <int D, int DPT>
 constexpr int f32_tpr() {
-  return D / DPT;  // lanes per row
+  return D / kF32Dpt;  // lanes per row
 }
-// KG groups per row (wide form): the row's keys (forward, dQ) or queries
-// (dK/dV) are dealt out to KG groups of TPR lanes, each keeping its own
-// softmax state or partial sums, merged at the end of the row pass.  Rows
-// per pass: up to 512 threads per group.
-template <int D, int DPT>
-constexpr int f32_rows() {
-  return kF32WgRows * f32_tpr<D, DPT>() <= 512 ? kF32WgRows : 512 / f32_tpr<D, DPT>();
+template <int D>
+constexpr int f32_rows() {  // rows per pass of at most 512 threads
+  return kF32WgRows * f32_tpr<D>() <= 512 ? kF32WgRows : 512 / f32_tpr<D>();
 }
-template <int D, int DPT, int KG = 1>
+template <int D>
 constexpr int f32_threads() {
-  return f32_rows<D, DPT>() * f32_tpr<D, DPT>() * KG;
+  return f32_rows<D>() * f32_tpr<D>();
 }
 
 // Sum over the TPR (1 to 16) consecutive lanes of one row, by the DPP steps
@@ -2027,13 +2004,12 @@ struct F32Stage {
   }
 };
 
-template <int D, bool CAUSAL, int DPT, int KG>
-__global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_fwd_f32_kernel(
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__((f32_threads<D>())) void attn_fwd_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     float* __restrict__ o, float* __restrict__ lse, ItemSource src, int tmax, int head_major,
     int heads, int group, Strides sq, Strides sk, Strides sv, Strides so, float scale, int total) {
-  constexpr int TPR = f32_tpr<D, DPT>(), RPP = f32_rows<D, DPT>(), KT = kF32Rows;
-  static_assert(KT % KG == 0 && (KG == 1 || KG == 2), "one or two key groups");
+  constexpr int DPT = kF32Dpt, TPR = f32_tpr<D>(), RPP = f32_rows<D>(), KT = kF32Rows;
   __shared__ __align__(16) float sK[KT * D];
   __shared__ __align__(16) float sV[KT * D];
   const ItemView iv = item_view<true>(src, tmax);
@@ -2058,10 +2034,9 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_fwd_f32_kern
     const float* kh = k + (int64_t)start * sk.row + (int64_t)hk * sk.head;
     const float* vh = v + (int64_t)start * sv.row + (int64_t)hk * sv.head;
     const int kend = CAUSAL ? min(L, q0 + kF32WgRows) : L;
-    const int kg = KG > 1 ? ((int)threadIdx.x / TPR) % KG : 0;  // this lane's key group
-    F32Stage<D, f32_threads<D, DPT, KG>()> stage;
+    F32Stage<D, f32_threads<D>()> stage;
     for (int r0 = 0; r0 < kF32WgRows && q0 + r0 < L; r0 += RPP) {
-      const int my_q = q0 + r0 + (int)threadIdx.x / (TPR * KG);
+      const int my_q = q0 + r0 + (int)threadIdx.x / TPR;
       // rows past L compute on row L-1 and store nothing
       float qv[DPT], ov[DPT];
       load_slice(qv, q + (int64_t)(start + min(my_q, L - 1)) * sq.row + (int64_t)h * sq.head + c0);
@@ -2076,31 +2051,26 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_fwd_f32_kern
         stage.store(sK, sV);
         __syncthreads();
         if (kb + KT < kpass) stage.load(kh, sk.row, vh, sv.row, kb + KT, kend);
-        float s[KT / KG];  // this group's keys of the tile: kg, kg + KG, ...
+        float s[KT];
         float tile_m = kNegInf;
 #pragma unroll
-        for (int j = 0; j < KT / KG; ++j) {
-          const int i = j * KG + kg;
+        for (int i = 0; i < KT; ++i) {
           float kr[DPT];
           load_slice(kr, sK + i * D + c0);
           const float dotv = row_sum<TPR>(dot_slice(qv, kr)) * scale;
-          s[j] = kb + i <= qlim ? dotv : kNegInf;
-          tile_m = fmaxf(tile_m, s[j]);
+          s[i] = kb + i <= qlim ? dotv : kNegInf;
+          tile_m = fmaxf(tile_m, s[i]);
         }
-        // key 0 is in every row's first tile, so m is finite from then on;
-        // with two key groups the second may see no key of a row at all
-        // (row 0, or a length-1 sequence): its m stays -inf, its weights 0
-        const float m_new = fmaxf(m, tile_m);
-        const float m_ref = KG > 1 && m_new == kNegInf ? 0.f : m_new;
-        const float alpha = fast_exp2((m - m_ref) * kLog2e);
+        const float m_new = fmaxf(m, tile_m);  // key 0 is in every row's first tile
+        const float alpha = fast_exp2((m - m_new) * kLog2e);
         float ot[DPT], lt = 0.f;
 #pragma unroll
         for (int d = 0; d < DPT; ++d) ot[d] = 0.f;
 #pragma unroll 4
-        for (int j = 0; j < KT / KG; ++j) {
-          const float p = fast_exp2((s[j] - m_ref) * kLog2e);
+        for (int i = 0; i < KT; ++i) {
+          const float p = fast_exp2((s[i] - m_new) * kLog2e);
           float vr[DPT];
-          load_slice(vr, sV + (j * KG + kg) * D + c0);
+          load_slice(vr, sV + i * D + c0);
           lt += p;
           axpy_slice(ot, p, vr);
         }
@@ -2109,19 +2079,7 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_fwd_f32_kern
         for (int d = 0; d < DPT; ++d) ov[d] = fmaf(ov[d], alpha, ot[d]);
         m = m_new;
       }
-      if constexpr (KG > 1) {  // merge the two groups' states (lanes TPR apart)
-        const float m_all = fmaxf(m, __shfl_xor(m, TPR, kWave));  // group 0 holds key 0: finite
-        const float a = fast_exp2((m - m_all) * kLog2e);
-        l *= a;
-        l += __shfl_xor(l, TPR, kWave);
-#pragma unroll
-        for (int d = 0; d < DPT; ++d) {
-          ov[d] *= a;
-          ov[d] += __shfl_xor(ov[d], TPR, kWave);
-        }
-        m = m_all;
-      }
-      if (my_q < L && kg == 0) {
+      if (my_q < L) {
         store_slice(o + (int64_t)(start + my_q) * so.row + (int64_t)h * so.head + c0, ov, 1.0f / l);
         if (c0 == 0) lse[(int64_t)(start + my_q) * heads + h] = m + logf(l);
       }
@@ -2133,15 +2091,14 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_fwd_f32_kern
 
 // dQ = scale * dS K with dS = P (dP - Delta), P = exp(S - LSE), dP = dO V^T;
 // Delta = rowsum(O * dO) is formed here and written out for the dK/dV pass.
-template <int D, bool CAUSAL, int DPT, int KG>
-__global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dq_f32_kernel(
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__((f32_threads<D>())) void attn_bwd_dq_f32_kernel(
     const float* __restrict__ dout, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ lse,
     float* __restrict__ delta, float* __restrict__ dq, ItemSource src, int tmax, int head_major,
     int heads, int group, Strides sdo, Strides sq, Strides sk, Strides sv, Strides so,
     Strides sdq, float scale, int total) {
-  constexpr int TPR = f32_tpr<D, DPT>(), RPP = f32_rows<D, DPT>(), KT = kF32Rows;
-  static_assert(KT % KG == 0 && (KG == 1 || KG == 2), "one or two key groups");
+  constexpr int DPT = kF32Dpt, TPR = f32_tpr<D>(), RPP = f32_rows<D>(), KT = kF32Rows;
   __shared__ __align__(16) float sK[KT * D];
   __shared__ __align__(16) float sV[KT * D];
   const ItemView iv = item_view<false>(src, tmax);
@@ -2164,10 +2121,9 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dq_f32_k
   const float* vh = v + (int64_t)start * sv.row + (int64_t)hk * sv.head;
   const int kend = CAUSAL ? min(L, q0 + kF32WgRows) : L;
   const float c = scale * kLog2e;
-  const int kg = KG > 1 ? ((int)threadIdx.x / TPR) % KG : 0;  // this lane's key group
-  F32Stage<D, f32_threads<D, DPT, KG>()> stage;
+  F32Stage<D, f32_threads<D>()> stage;
   for (int r0 = 0; r0 < kF32WgRows && q0 + r0 < L; r0 += RPP) {
-    const int my_q = q0 + r0 + (int)threadIdx.x / (TPR * KG);
+    const int my_q = q0 + r0 + (int)threadIdx.x / TPR;
     const int64_t tok = start + min(my_q, L - 1);
     const int kpass = CAUSAL ? min(kend, q0 + r0 + RPP) : kend;
     stage.load(kh, sk.row, vh, sv.row, 0, kend);
@@ -2180,7 +2136,7 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dq_f32_k
       load_slice(ov, o + tok * so.row + (int64_t)h * so.head + c0);
       dl = row_sum<TPR>(dot_slice(ov, dov));
     }
-    if (my_q < L && c0 == 0 && kg == 0) delta[(int64_t)(start + my_q) * heads + h] = dl;
+    if (my_q < L && c0 == 0) delta[(int64_t)(start + my_q) * heads + h] = dl;
     const float lse2 = lse[tok * heads + h] * kLog2e;
 #pragma unroll
     for (int d = 0; d < DPT; ++d) dqv[d] = 0.f;
@@ -2194,8 +2150,7 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dq_f32_k
 #pragma unroll
       for (int d = 0; d < DPT; ++d) dqt[d] = 0.f;
 #pragma unroll 2
-      for (int j = 0; j < KT / KG; ++j) {  // this group's keys: kg, kg + KG, ...
-        const int i = j * KG + kg;
+      for (int i = 0; i < KT; ++i) {
         float kr[DPT], vr[DPT];
         load_slice(kr, sK + i * D + c0);
         load_slice(vr, sV + i * D + c0);
@@ -2207,26 +2162,21 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dq_f32_k
 #pragma unroll
       for (int d = 0; d < DPT; ++d) dqv[d] += dqt[d];
     }
-    if constexpr (KG > 1) {  // the two groups' sums (lanes TPR apart)
-#pragma unroll
-      for (int d = 0; d < DPT; ++d) dqv[d] += __shfl_xor(dqv[d], TPR, kWave);
-    }
-    if (my_q < L && kg == 0)
+    if (my_q < L)
       store_slice(dq + (int64_t)(start + my_q) * sdq.row + (int64_t)h * sdq.head + c0, dqv, scale);
   }
 }
 
 // dV = P^T dO and dK = scale * dS^T Q for 64 of an item's keys, summed over
 // the query heads that share their K/V head.
-template <int D, bool CAUSAL, int DPT, int KG>
-__global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dkv_f32_kernel(
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__((f32_threads<D>())) void attn_bwd_dkv_f32_kernel(
     const float* __restrict__ dout, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ lse, const float* __restrict__ delta,
     float* __restrict__ dk, float* __restrict__ dv, ItemSource src, int tmax, int head_major,
     int kv_heads, int group, Strides sdo, Strides sq, Strides sk, Strides sv, Strides sdk,
     Strides sdv, float scale, int total) {
-  constexpr int TPR = f32_tpr<D, DPT>(), RPP = f32_rows<D, DPT>(), QT = kF32Rows;
-  static_assert(QT % KG == 0 && (KG == 1 || KG == 2), "one or two query groups");
+  constexpr int DPT = kF32Dpt, TPR = f32_tpr<D>(), RPP = f32_rows<D>(), QT = kF32Rows;
   __shared__ __align__(16) float sQ[QT * D];
   __shared__ __align__(16) float sO[QT * D];  // dO rows
   __shared__ float sL[QT], sD[QT];             // LSE * log2(e) and Delta of those rows
@@ -2249,10 +2199,9 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dkv_f32_
   const int heads = kv_heads * group;
   const int c0 = (threadIdx.x % TPR) * DPT;
   const float c = scale * kLog2e;
-  const int kg = KG > 1 ? ((int)threadIdx.x / TPR) % KG : 0;  // this lane's query group
-  F32Stage<D, f32_threads<D, DPT, KG>()> stage;
+  F32Stage<D, f32_threads<D>()> stage;
   for (int r0 = 0; r0 < kF32WgRows && k0 + r0 < L; r0 += RPP) {
-    const int my_k = k0 + r0 + (int)threadIdx.x / (TPR * KG);
+    const int my_k = k0 + r0 + (int)threadIdx.x / TPR;
     const int64_t tok = start + min(my_k, L - 1);
     float kv[DPT], vv[DPT], dkv[DPT], dvv[DPT];
     load_slice(kv, k + tok * sk.row + (int64_t)hk * sk.head + c0);
@@ -2288,8 +2237,7 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dkv_f32_
 #pragma unroll
         for (int d = 0; d < DPT; ++d) dkt[d] = dvt[d] = 0.f;
 #pragma unroll 2
-        for (int j = 0; j < QT / KG; ++j) {  // this group's queries: kg, kg + KG, ...
-          const int i = j * KG + kg;
+        for (int i = 0; i < QT; ++i) {
           const int qq = qb + i;
           float qr[DPT], orow[DPT];
           load_slice(qr, sQ + i * D + c0);
@@ -2308,18 +2256,629 @@ __global__ __launch_bounds__((f32_threads<D, DPT, KG>())) void attn_bwd_dkv_f32_
         }
       }
     }
-    if constexpr (KG > 1) {  // the two groups' sums (lanes TPR apart)
-#pragma unroll
-      for (int d = 0; d < DPT; ++d) {
-        dkv[d] += __shfl_xor(dkv[d], TPR, kWave);
-        dvv[d] += __shfl_xor(dvv[d], TPR, kWave);
-      }
-    }
-    if (my_k < L && kg == 0) {
+    if (my_k < L) {
       store_slice(dk + (int64_t)(start + my_k) * sdk.row + (int64_t)hk * sdk.head + c0, dkv, scale);
       store_slice(dv + (int64_t)(start + my_k) * sdv.row + (int64_t)hk * sdv.head + c0, dvv, 1.0f);
     }
   }
+}
+
+// ------------------------------------------- fp32 on the matrix instructions
+// fp32 inputs, which the reference's Array-level function computes as given
+// (its torch branch, reference/varlen_attention.py:90-113), on
+// v_mfma_f32_32x32x2_f32: fp32 operands, products and sums throughout.  A
+// 32x32 score tile at head_dim 64 is 32 of these (64 cycles each) against
+// ~300 cycles of softmax arithmetic, so the kernels are bound by the matrix
+// cores (154 TFLOP/s measured for a large fp32 GEMM on this GPU); FP32 FMAs
+// with operands from LDS, which they replace, reached 12-30 TFLOP/s.
+//
+// Operand layout.  An instruction takes k = 2: lane (r = l % 32, g = l / 32)
+// supplies A[r][g] and B[g][r], and which k index "g" is, is free as long as
+// both operands agree.  So
+//  * row operands (K, Q, V, dO rows against D): lane (r, g) holds 16-byte
+//    fragments [8j + 4g, 8j + 4g + 4) of row r; fragment j feeds four k-steps;
+//  * the score tile's accumulator (element i of lane (r, g): row
+//    8*(i/4) + 4g + i%4, column r) is the B operand of the next product as it
+//    stands: k-step t takes element t, i.e. rows 8*(t/4) + t%4 and + 4;
+//  * column operands (V^T, K^T, dO^T, Q^T): at k-step t lane (r, g) holds ND =
+//    D / 32 adjacent columns ND*r .. of row 8*(t/4) + 4g + t%4, one for each
+//    of the ND output tiles, so output tile dt covers columns ND*m + dt and
+//    every load is a contiguous run of whole rows.
+// Operands come from the L1 / L2 straight into registers (16 bytes per lane
+// feed 256 cycles of MFMA; no LDS tile, no barrier in the loop); the loads of
+// one phase are issued a whole phase (D / 2 MFMAs) ahead into one of two
+// buffers.  Buffer descriptors cover the sequence's valid rows only: rows
+// past it read as zeros.
+//
+// KG of the four waves of a workgroup share 32 rows and deal the tiles they
+// sweep out among themselves (their results merge through LDS in wave order),
+// so a workgroup holds 128 / KG rows of an item: KG = 4 or 2 for small
+// launches, where a row block's chain of tiles is what takes the time, KG = 1
+// for large ones (f32m_share).
+//
+// Measured (16 sequences of mean 256, 8 heads of 64, causal; the FMA kernels
+// before): forward 115 -> 38 us, dQ 109 -> 49, dK/dV 159 -> 63; two sequences
+// of 4,096: 811 -> 337, 810 -> 483, 1,390 -> 654 us (102-107 TFLOP/s of the
+// executed products).
+//
+// Rounding: a dot product over D is summed in chunks of 16 columns (8 columns
+// at KG = 4) and then over the chunks in pairs, and every sum over keys or
+// queries per half tile of 16 rows, then over the halves and the tiles.  The
+// error against 64 bits (2-norm, 28 problems over head_dim 32-128, 256-8,192
+// tokens) is 0.95 / 0.99 / 0.96 / 0.93 of the FMA kernels' (out, dQ, dK, dV;
+// geometric means); with one chain per 32-row tile and 16-column chunks
+// throughout it was 1.02 / 1.01 / 0.98 / 0.96, 3-5 % faster at head_dim 64.
+__device__ __forceinline__ f32x16 mfma2(float a, float b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+template <int D>
+constexpr int f32m_nd() {  // output tiles: columns per lane of a column operand
+  return D >= 32 ? D / 32 : 1;
+}
+template <int KG>
+constexpr int f32m_chunk() {  // row fragments per chunk of a dot product
+  return KG == 4 ? 1 : 2;
+}
+template <int D>
+constexpr int f32m_buf() {  // floats per lane of one 32-row tile, either form
+  return 16 * f32m_nd<D>() > D / 2 ? 16 * f32m_nd<D>() : D / 2;
+}
+constexpr int kF32Pad = 4;  // LDS rows of D + 4 floats: 16 rows' chunks fall on distinct banks
+
+// Loads of 32-row tiles of a (rows, D) matrix.
+template <int D>
+struct F32Tile {
+  static constexpr int ND = f32m_nd<D>();
+  uint32_t vrow;     // byte offset of row r, column 4g
+  uint32_t vcol[4];  // byte offset of row 4g + e, column ND*r
+  int64_t stride;    // elements per row
+  __device__ __forceinline__ void init(int64_t row_stride, int r, int g) {
+    stride = row_stride;
+    vrow = (uint32_t)((r * row_stride + 4 * g) * 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)  // head_dim 16: lanes past its columns read zeros
+      vcol[e] = ND * r < D ? (uint32_t)(((4 * g + e) * row_stride + ND * r) * 4) : 0xFFFFFFF0u;
+  }
+  // bytes of rows [row0, row0 + n) that the sequence of `limit` rows holds
+  __device__ __forceinline__ uint32_t bytes(int row0, int n, int limit) const {
+    const int valid = min(n, limit - row0);
+    return valid > 0 ? (uint32_t)(((valid - 1) * stride + D) * 4) : 0u;
+  }
+  __device__ __forceinline__ void rows(float (&b)[f32m_buf<D>()], const float* __restrict__ base,
+                                       int row0, int limit) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + (int64_t)row0 * stride, bytes(row0, 32, limit));
+    uint32_t vr = vrow;
+    asm volatile("" : "+v"(vr));  // keeps the +32j in the instructions' offsets, not in registers of their own
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) {
+      const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, vr + 32 * j, 0, 0));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) b[4 * j + e] = v[e];
+    }
+#else
+    (void)b, (void)base, (void)row0, (void)limit;
+#endif
+  }
+  __device__ __forceinline__ void cols(float (&b)[f32m_buf<D>()], const float* __restrict__ base,
+                                       int row0, int limit) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const __amdgpu_buffer_rsrc_t rs =
+          make_rsrc(base + (int64_t)(row0 + 8 * j) * stride, bytes(row0 + 8 * j, 8, limit));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = ND * (4 * j + e);
+        if constexpr (ND == 4) {
+          const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, vcol[e], 0, 0));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) b[t + i] = v[i];
+        } else if constexpr (ND == 2) {
+          typedef float f32x2 __attribute__((ext_vector_type(2)));
+          const f32x2 v = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, vcol[e], 0, 0));
+          b[t] = v[0];
+          b[t + 1] = v[1];
+        } else {
+          b[t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, vcol[e], 0, 0));
+        }
+      }
+    }
+#else
+    (void)b, (void)base, (void)row0, (void)limit;
+#endif
+  }
+};
+
+// A 32x32 tile of row-operand products over D: `a` in registers, fragment j
+// of the other operand from frag(j).  Chunks of FR fragments (8 FR columns),
+// summed in pairs.
+// (The scheduling barrier and the empty asm per chunk: left alone the compiler
+// runs every chunk's chain side by side, 16 registers each, sinks the sums to
+// their use, and spills.)
+template <int D, int FR, typename Frag>
+__device__ __forceinline__ f32x16 f32m_dot(const float (&a)[f32m_buf<D>()], Frag frag) {
+  constexpr int NC = D / (8 * FR);
+  f32x16 s, pair, prev;
+#pragma unroll
+  for (int c = 0; c <= NC; ++c) {
+    f32x16 acc;
+    if (c < NC) {
+      acc = zero16();
+#pragma unroll
+      for (int jj = 0; jj < FR; ++jj) {
+        const float4 f = frag(FR * c + jj);
+        const float fe[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = mfma2(a[4 * (FR * c + jj) + e], fe[e], acc);
+      }
+    }
+    if (c > 0) {  // fold in chunk c - 1 while this one's instructions run
+      if (c % 2 == 1) {
+        pair = prev;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pair[i] += prev[i];
+        asm volatile("" : "+v"(pair));
+      }
+      if (c == 2 || NC == 1) s = pair;
+      if (c > 2 && c % 2 == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] += pair[i];
+        asm volatile("" : "+v"(s));
+      }
+    }
+    if (c < NC) prev = acc;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return s;
+}
+template <int D>
+__device__ __forceinline__ float4 f32m_frag(const float (&b)[f32m_buf<D>()], int j) {
+  return make_float4(b[4 * j], b[4 * j + 1], b[4 * j + 2], b[4 * j + 3]);
+}
+
+// One tile's column-operand product: acc[dt] = fma(acc[dt], alpha, tile sum).
+template <int D>
+__device__ __forceinline__ void f32m_accum(f32x16 (&acc)[f32m_nd<D>()], float alpha,
+                                           const float (&a)[f32m_buf<D>()], const f32x16& b) {
+  constexpr int ND = f32m_nd<D>();
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt) {
+    f32x16 t = zero16(), u = zero16();
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t = mfma2(a[ND * k + dt], b[k], t);
+#pragma unroll
+    for (int k = 8; k < 16; ++k) u = mfma2(a[ND * k + dt], b[k], u);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[dt][i] = fmaf(acc[dt][i], alpha, t[i] + u[i]);
+    asm volatile("" : "+v"(acc[dt]));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// This wave's 32 output rows (lane r's row, times `mul`) into its LDS area.
+template <int D>
+__device__ __forceinline__ void f32m_stage(float* stage, const f32x16 (&acc)[f32m_nd<D>()], float mul,
+                                           int r, int g) {
+  constexpr int ND = f32m_nd<D>();
+#pragma unroll
+  for (int qd = 0; qd < 4; ++qd) {
+    const int c0 = ND * (8 * qd + 4 * g);  // elements 4qd .. 4qd+3 of the ND tiles: 4*ND columns from here
+    if (c0 >= D) continue;                 // head_dim 16
+    float f[4 * ND];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) f[e * ND + dt] = acc[dt][4 * qd + e] * mul;
+    store_slice(stage + r * (D + kF32Pad) + c0, f, 1.0f);
+  }
+}
+// The workgroup's rows from the staged areas, the KG waves of a row tile
+// added in wave order, as contiguous row stores.  Rows >= nrows are not stored.
+template <int D, int KG>
+__device__ __forceinline__ void f32m_store(const float* stage, float* __restrict__ dst,
+                                           int64_t row_stride, int nrows) {
+  constexpr int C4 = D / 4, SD = D + kF32Pad;
+  for (int idx = threadIdx.x; idx < (4 / KG) * 32 * C4; idx += kThreads) {
+    const int row = idx / C4, c = 4 * (idx % C4);
+    if (row >= nrows) break;
+    const float* p = stage + ((row >> 5) * KG * 32 + (row & 31)) * SD + c;
+    float4 s = *reinterpret_cast<const float4*>(p);
+#pragma unroll
+    for (int j = 1; j < KG; ++j) {
+      const float4 x = *reinterpret_cast<const float4*>(p + j * 32 * SD);
+      s.x += x.x, s.y += x.y, s.z += x.z, s.w += x.w;
+    }
+    *reinterpret_cast<float4*>(dst + (int64_t)row * row_stride + c) = s;
+  }
+}
+
+// Block -> (logical block, part of the item's rows): the parts of an (item,
+// head) are KG blocks apart by 8, so they run on the XCD that map_block_at
+// assumes for the logical block.  The grid is whole groups of 8 * KG.
+template <int KG>
+__device__ __forceinline__ void f32m_block(int& b, int& part) {
+  const int x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+  part = j % KG;
+  b = (j / KG) * kXcds + x;
+}
+
+template <int D>
+constexpr int f32m_waves() {  // waves per SIMD: the buffers and accumulators of head_dim 128 need one's registers
+  return D <= 64 ? 2 : 1;
+}
+
+// A wave's own row operands (Q; Q and dO; K and V) stay in registers where
+// these hold them beside the buffers and accumulators, else in LDS rows (one
+// copy for the KG waves of a row tile).
+template <int D, int KG>
+__device__ __forceinline__ void f32m_put(float* lds, const float (&b)[f32m_buf<D>()], int kg) {
+#pragma unroll
+  for (int j = 0; j < D / 8; ++j)
+    if (j % KG == kg) *reinterpret_cast<float4*>(lds + 8 * j) = f32m_frag<D>(b, j);
+}
+
+template <int D, bool CAUSAL, int KG>
+__global__ __launch_bounds__(kThreads, (D == 64 && KG == 2 ? 3 : f32m_waves<D>())) void attn_fwd_f32m_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    float* __restrict__ o, float* __restrict__ lse, ItemSource src, int tmax, int head_major,
+    int heads, int group, Strides sq, Strides sk, Strides sv, Strides so, float scale, int total) {
+  constexpr int ND = f32m_nd<D>(), NB = f32m_buf<D>(), SD = D + kF32Pad;
+  __shared__ __align__(16) float stage[4 * 32 * SD];
+  __shared__ float s_m[4][32], s_l[4][32];
+  const ItemView iv = item_view<true>(src, tmax);
+  if (iv.failed) {
+    publish_header(src, iv, CAUSAL ? 1 : 0);
+    poison_rows(o, so, total, heads, D);
+    poison_stats(lse, total, heads);
+    return;
+  }
+  int b, part, item, h;
+  f32m_block<KG>(b, part);
+  if (!map_block_at(b, heads, tmax, head_major, group, false, item, h) || item >= iv.count) {
+    publish_header(src, iv, CAUSAL ? 1 : 0);
+    return;
+  }
+  const int4 it = item_at<true>(src, iv, CAUSAL, item);
+  const int start = it.z, L = it.w, q0 = it.y * kBM + part * (kBM / KG);  // this workgroup's rows
+  if (L > 0 && q0 < L) {
+    const int hk = h / group;
+    const float scale_log2 = scale * kLog2e;
+    const int wave = wave_id(), lane = threadIdx.x & (kWave - 1), r = lane & 31, g = lane >> 5;
+    const int kg = wave % KG, qw0 = q0 + 32 * (wave / KG);
+    f32x16 oacc[ND];
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) oacc[dt] = zero16();
+    float m = kNegInf, l = 0.f;
+    constexpr bool kQLds = D >= 128 || (D == 64 && KG == 2);  // three waves per SIMD at 64
+    float qv[NB];
+    float* ql = stage + (wave / KG) * 32 * SD + r * SD + 4 * g;  // (the stage holds O only after the loop)
+    {
+      F32Tile<D> t;
+      t.init(sq.row, r, g);
+      t.rows(qv, q + (int64_t)start * sq.row + (int64_t)h * sq.head, qw0, L);
+    }
+    if constexpr (kQLds) {
+      f32m_put<D, KG>(ql, qv, kg);
+      __syncthreads();
+    }
+    auto qfrag = [&](int j) {
+      if constexpr (kQLds) return *reinterpret_cast<const float4*>(ql + 8 * j);
+      else return f32m_frag<D>(qv, j);
+    };
+    if (qw0 < L) {
+      const float* kh = k + (int64_t)start * sk.row + (int64_t)hk * sk.head;
+      const float* vh = v + (int64_t)start * sv.row + (int64_t)hk * sv.head;
+      const int nt = CAUSAL ? qw0 / 32 + 1 : (L + 31) / 32;
+      F32Tile<D> tk, tv;
+      tk.init(sk.row, r, g);
+      tv.init(sv.row, r, g);
+      float X[NB], Y[NB];
+      if (kg < nt) tk.rows(X, kh, 32 * kg, L);
+      for (int kt = kg; kt < nt; kt += KG) {
+        tv.cols(Y, vh, 32 * kt, L);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 s = f32m_dot<D, f32m_chunk<KG>()>(X, qfrag);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + KG < nt) tk.rows(X, kh, 32 * (kt + KG), L);
+        __builtin_amdgcn_sched_barrier(0);
+        // scores in units of log2(e); the largest weight of a row is exactly 1
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] *= scale_log2;
+        if (CAUSAL) {
+          if (32 * kt == qw0) mask_rows_above<false>(s, r - 4 * g);  // the diagonal tile
+        } else if (32 * kt + 32 > L) {
+          mask_rows_above<false>(s, L - 1 - 32 * kt - 4 * g);
+        }
+        // a tile whose scores are all -inf for a row leaves its m at -inf
+        const float m_new = fmaxf(m, tile_max_fresh(s));
+        const float m_ref = m_new == kNegInf ? 0.f : m_new;
+        const float alpha = fast_exp2(m - m_ref);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = fast_exp2(s[i] - m_ref);
+        l = fmaf(l, alpha, tile_sum(s));
+        m = m_new;
+        f32m_accum<D>(oacc, alpha, Y, s);
+      }
+    }
+    // merge the KG waves of each row tile: weights relative to the rows' maximum
+    float l_all = halves_sum(l), m_all = m, a = 1.0f;
+    if constexpr (KG > 1) {
+      s_m[wave][r] = m;
+      s_l[wave][r] = l_all;
+      __syncthreads();
+      const int w0 = wave - kg;
+#pragma unroll
+      for (int j = 0; j < KG; ++j) m_all = fmaxf(m_all, s_m[w0 + j][r]);
+      l_all = 0.f;
+#pragma unroll
+      for (int j = 0; j < KG; ++j) l_all = fmaf(s_l[w0 + j][r], fast_exp2(s_m[w0 + j][r] - m_all), l_all);
+      a = fast_exp2(m - m_all);
+    }
+    if constexpr (kQLds) __syncthreads();  // every wave is done with the staged Q rows
+    f32m_stage<D>(stage + wave * 32 * SD, oacc, a / l_all, r, g);
+    if (kg == 0 && g == 0 && qw0 + r < L)
+      lse[(int64_t)(start + qw0 + r) * heads + h] = fmaf(m_all, kLn2, logf(l_all));
+    __syncthreads();
+    f32m_store<D, KG>(stage, o + (int64_t)(start + q0) * so.row + (int64_t)h * so.head, so.row, L - q0);
+  }
+  publish_header(src, iv, CAUSAL ? 1 : 0);
+  if (h == 0 && part == 0 && L > 0) publish_item(src, item, it);
+}
+
+// dQ = scale * dS K with dS = P (dP - Delta), P = exp(S - LSE), dP = dO V^T;
+// Delta = rowsum(O * dO) is formed here and written out for the dK/dV pass.
+// The scores are transposed (keys x queries), as in the forward.
+template <int D>
+constexpr bool f32m_op_lds() {  // backward: two row operands per wave
+  return D >= 64;
+}
+template <int D, bool CAUSAL, int KG>
+__global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dq_f32m_kernel(
+    const float* __restrict__ dout, const float* __restrict__ q, const float* __restrict__ k,
+    const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ lse,
+    float* __restrict__ delta, float* __restrict__ dq, ItemSource src, int tmax, int head_major,
+    int heads, int group, Strides sdo, Strides sq, Strides sk, Strides sv, Strides so,
+    Strides sdq, float scale, int total) {
+  constexpr int ND = f32m_nd<D>(), NB = f32m_buf<D>(), SD = D + kF32Pad, RT = 4 / KG;
+  constexpr int OPF = f32m_op_lds<D>() ? RT * 2 * 32 * SD : 0, STF = 4 * 32 * SD;
+  __shared__ __align__(16) float smem[OPF > STF ? OPF : STF];
+  const ItemView iv = item_view<false>(src, tmax);
+  if (iv.failed) {
+    poison_rows(dq, sdq, total, heads, D);
+    poison_stats(delta, total, heads);
+    return;
+  }
+  int b, part, item, h;
+  f32m_block<KG>(b, part);
+  if (!map_block_at(b, heads, tmax, head_major, group, false, item, h) || item >= iv.count) return;
+  const int4 it = item_at<false>(src, iv, CAUSAL, item);
+  const int start = it.z, L = it.w, q0 = it.y * kBM + part * (kBM / KG);
+  if (L == 0 || q0 >= L) return;
+  const int hk = h / group;
+  const int wave = wave_id(), lane = threadIdx.x & (kWave - 1), r = lane & 31, g = lane >> 5;
+  const int kg = wave % KG, qw0 = q0 + 32 * (wave / KG);
+  f32x16 dqacc[ND];
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt) dqacc[dt] = zero16();
+  float qv[NB], dov[NB], X[NB];
+  float dl, lse2;
+  {
+    F32Tile<D> t;
+    t.init(so.row, r, g);
+    t.rows(X, o + (int64_t)start * so.row + (int64_t)h * so.head, qw0, L);
+    t.init(sdo.row, r, g);
+    t.rows(dov, dout + (int64_t)start * sdo.row + (int64_t)h * sdo.head, qw0, L);
+    t.init(sq.row, r, g);
+    t.rows(qv, q + (int64_t)start * sq.row + (int64_t)h * sq.head, qw0, L);
+    lse2 = lse[(int64_t)(start + min(qw0 + r, L - 1)) * heads + h] * kLog2e;
+    float d[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < D / 2; ++i) d[i & 3] = fmaf(X[i], dov[i], d[i & 3]);
+    dl = halves_sum((d[0] + d[1]) + (d[2] + d[3]));
+    if (kg == 0 && g == 0 && qw0 + r < L) delta[(int64_t)(start + qw0 + r) * heads + h] = dl;
+  }
+  float* ql = smem + (wave / KG) * 2 * 32 * SD + r * SD + 4 * g;  // this lane's fragments of Q, then dO
+  float* dol = ql + 32 * SD;
+  if constexpr (f32m_op_lds<D>()) {
+    f32m_put<D, KG>(ql, qv, kg);
+    f32m_put<D, KG>(dol, dov, kg);
+    __syncthreads();
+  }
+  auto qfrag = [&](int j) {
+    if constexpr (f32m_op_lds<D>()) return *reinterpret_cast<const float4*>(ql + 8 * j);
+    else return f32m_frag<D>(qv, j);
+  };
+  auto dofrag = [&](int j) {
+    if constexpr (f32m_op_lds<D>()) return *reinterpret_cast<const float4*>(dol + 8 * j);
+    else return f32m_frag<D>(dov, j);
+  };
+  const int nt = CAUSAL ? qw0 / 32 + 1 : (L + 31) / 32;
+  if (qw0 < L && kg < nt) {
+    const float* kh = k + (int64_t)start * sk.row + (int64_t)hk * sk.head;
+    const float* vh = v + (int64_t)start * sv.row + (int64_t)hk * sv.head;
+    const float c = scale * kLog2e;
+    F32Tile<D> tk, tv;
+    tk.init(sk.row, r, g);
+    tv.init(sv.row, r, g);
+    float Y[NB], Z[NB];
+    tk.rows(X, kh, 32 * kg, L);
+    tv.rows(Y, vh, 32 * kg, L);
+    for (int kt = kg; kt < nt; kt += KG) {
+      const bool more = kt + KG < nt;
+      tk.cols(Z, kh, 32 * kt, L);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 s = f32m_dot<D, f32m_chunk<KG>()>(X, qfrag);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) tk.rows(X, kh, 32 * (kt + KG), L);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 dp = f32m_dot<D, f32m_chunk<KG>()>(Y, dofrag);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) tv.rows(Y, vh, 32 * (kt + KG), L);
+      __builtin_amdgcn_sched_barrier(0);
+      if (CAUSAL) {
+        if (32 * kt == qw0) mask_rows_above<false>(s, r - 4 * g);
+      } else if (32 * kt + 32 > L) {
+        mask_rows_above<false>(s, L - 1 - 32 * kt - 4 * g);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = fast_exp2(fmaf(s[i], c, -lse2)) * (dp[i] - dl);
+      f32m_accum<D>(dqacc, 1.0f, Z, s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (f32m_op_lds<D>()) __syncthreads();  // every wave is done with the staged rows
+  float* stage = smem;
+  f32m_stage<D>(stage + wave * 32 * SD, dqacc, scale, r, g);
+  __syncthreads();
+  f32m_store<D, KG>(stage, dq + (int64_t)(start + q0) * sdq.row + (int64_t)h * sdq.head, sdq.row, L - q0);
+}
+
+// dV = P^T dO and dK = scale * dS^T Q for 128 / KG of an item's keys, summed
+// over the query heads that share their K/V head.  The wave's K and V rows
+// are staged in LDS from head_dim 64 up (in registers with the rest they
+// would spill), the waves of a row tile sharing one copy.
+template <int D, bool CAUSAL, int KG>
+__global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dkv_f32m_kernel(
+    const float* __restrict__ dout, const float* __restrict__ q, const float* __restrict__ k,
+    const float* __restrict__ v, const float* __restrict__ lse, const float* __restrict__ delta,
+    float* __restrict__ dk, float* __restrict__ dv, ItemSource src, int tmax, int head_major,
+    int kv_heads, int group, Strides sdo, Strides sq, Strides sk, Strides sv, Strides sdk,
+    Strides sdv, float scale, int total) {
+  constexpr int ND = f32m_nd<D>(), NB = f32m_buf<D>(), SD = D + kF32Pad, RT = 4 / KG;
+  constexpr int KVF = f32m_op_lds<D>() ? RT * 2 * 32 * SD : 0, STF = 4 * 32 * SD;
+  __shared__ __align__(16) float smem[KVF > STF ? KVF : STF];
+  __shared__ __align__(16) float s_rows[4][64];  // per wave: LSE * log2(e), then Delta, of a tile's queries
+  const ItemView iv = item_view<false>(src, tmax);
+  if (iv.failed) {
+    poison_rows(dk, sdk, total, kv_heads, D);
+    poison_rows(dv, sdv, total, kv_heads, D);
+    return;
+  }
+  int b, part, item, hk;
+  f32m_block<KG>(b, part);
+  if (!map_block_at(b, kv_heads, tmax, head_major, 1, false, item, hk) || item >= iv.count) return;
+  const int4 it = item_at<false>(src, iv, CAUSAL, item);
+  const int start = it.z, L = it.w;
+  const int nblk = (L + kBM - 1) / kBM;
+  const int k0 = (nblk - 1 - it.y) * kBM + part * (kBM / KG);  // key-major: the list's blk counts down
+  if (L == 0 || k0 >= L) return;
+  const int heads = kv_heads * group;
+  const int wave = wave_id(), lane = threadIdx.x & (kWave - 1), r = lane & 31, g = lane >> 5;
+  const int kg = wave % KG, rt = wave / KG, kw0 = k0 + 32 * rt;
+  const float c = scale * kLog2e;
+  f32x16 dkacc[ND], dvacc[ND];
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt) {
+    dkacc[dt] = zero16();
+    dvacc[dt] = zero16();
+  }
+  float kv[f32m_op_lds<D>() ? 1 : NB], vv[f32m_op_lds<D>() ? 1 : NB];
+  float* kl = smem + rt * 2 * 32 * SD + r * SD + 4 * g;  // this lane's fragments of K, then V
+  float* vl = kl + 32 * SD;
+  float X[NB], Y[NB];
+  {
+    F32Tile<D> t;
+    t.init(sk.row, r, g);
+    t.rows(X, k + (int64_t)start * sk.row + (int64_t)hk * sk.head, kw0, L);
+    t.init(sv.row, r, g);
+    t.rows(Y, v + (int64_t)start * sv.row + (int64_t)hk * sv.head, kw0, L);
+    if constexpr (f32m_op_lds<D>()) {
+      f32m_put<D, KG>(kl, X, kg);
+      f32m_put<D, KG>(vl, Y, kg);
+      __syncthreads();
+    } else {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        kv[i] = X[i];
+        vv[i] = Y[i];
+      }
+    }
+  }
+  auto kfrag = [&](int j) {
+    if constexpr (f32m_op_lds<D>()) return *reinterpret_cast<const float4*>(kl + 8 * j);
+    else return f32m_frag<D>(kv, j);
+  };
+  auto vfrag = [&](int j) {
+    if constexpr (f32m_op_lds<D>()) return *reinterpret_cast<const float4*>(vl + 8 * j);
+    else return f32m_frag<D>(vv, j);
+  };
+  const int qbeg = (CAUSAL ? kw0 : 0) + 32 * kg;  // this wave's first query tile of every head
+  if (kw0 < L && qbeg < L) {
+    F32Tile<D> tq, to;
+    tq.init(sq.row, r, g);
+    to.init(sdo.row, r, g);
+    int gi = 0, qb = qbeg;
+    const float* qh = q + (int64_t)start * sq.row + (int64_t)hk * group * sq.head;
+    const float* dh = dout + (int64_t)start * sdo.row + (int64_t)hk * group * sdo.head;
+    // lanes 0..31: LSE of query qb + lane; lanes 32..63: its Delta
+    auto row_stat = [&](int hh, int qq) {
+      const float* p = g ? delta : lse;
+      return qq < L ? p[(int64_t)(start + qq) * heads + hh] : 0.f;
+    };
+    float stat = row_stat(hk * group, qb + r);
+    tq.rows(X, qh, qb, L);
+    to.rows(Y, dh, qb, L);
+    float* rows = s_rows[wave];
+    while (true) {
+      rows[lane] = g ? stat : stat * kLog2e;
+      const int cur = qb;
+      const float* cqh = qh;
+      const float* cdh = dh;
+      qb += 32 * KG;
+      bool more = true;
+      if (qb >= L) {  // the group's next query head
+        qb = qbeg;
+        if (++gi == group) more = false;
+        qh += sq.head;
+        dh += sdo.head;
+      }
+      if (more) stat = row_stat(hk * group + gi, qb + r);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 s = f32m_dot<D, f32m_chunk<KG>()>(X, kfrag);
+      __builtin_amdgcn_sched_barrier(0);
+      to.cols(X, cdh, cur, L);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 dp = f32m_dot<D, f32m_chunk<KG>()>(Y, vfrag);
+      __builtin_amdgcn_sched_barrier(0);
+      tq.cols(Y, cqh, cur, L);
+      __builtin_amdgcn_sched_barrier(0);
+      if (CAUSAL && cur == kw0) mask_rows_below(s, r - 4 * g);  // queries before the key
+      if (cur + 32 > L) mask_rows_above(s, L - 1 - cur - 4 * g);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // this wave's own row statistics
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const float4 l4 = *reinterpret_cast<const float4*>(rows + 8 * i4 + 4 * g);
+        const float4 d4 = *reinterpret_cast<const float4*>(rows + 32 + 8 * i4 + 4 * g);
+        const float la[4] = {l4.x, l4.y, l4.z, l4.w}, da[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * i4 + e;
+          s[i] = fast_exp2(fmaf(s[i], c, -la[e]));
+          dp[i] = s[i] * (dp[i] - da[e]);
+        }
+      }
+      f32m_accum<D>(dvacc, 1.0f, X, s);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) tq.rows(X, qh, qb, L);
+      __builtin_amdgcn_sched_barrier(0);
+      f32m_accum<D>(dkacc, 1.0f, Y, dp);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!more) break;
+      to.rows(Y, dh, qb, L);
+    }
+  }
+  float* stage = smem + wave * 32 * SD;
+  __syncthreads();  // every wave is done with the staged K and V rows
+  f32m_stage<D>(stage, dkacc, scale, r, g);
+  __syncthreads();
+  f32m_store<D, KG>(smem, dk + (int64_t)(start + k0) * sdk.row + (int64_t)hk * sdk.head, sdk.row, L - k0);
+  __syncthreads();
+  f32m_stage<D>(stage, dvacc, 1.0f, r, g);
+  __syncthreads();
+  f32m_store<D, KG>(smem, dv + (int64_t)(start + k0) * sdv.row + (int64_t)hk * sdv.head, sdv.row, L - k0);
 }
 
 // ------------------------------------------------------------------- host
@@ -2535,114 +3094,100 @@ void launch_bwd_dkv_t(const void* dout, const void* q, const void* k, const void
     else { if (causal) FN<256, true>(__VA_ARGS__); else FN<256, false>(__VA_ARGS__); }           \
   } while (0)
 
-// The fp32 form for a grid: wide when the narrow form would give the GPU's
-// 1,024 SIMDs less than a wave each.
+// The waves that share a row tile in an fp32 launch of `blocks` (item, head)
+// pairs, four row tiles each: the tiles of a row block are dealt out over 4 or
+// 2 waves while one wave per row tile would leave the GPU's 1,024 SIMDs short
+// of work, since the longest row block's chain is then what takes the time;
+// past that the merge and the extra operand loads cost more than the shorter
+// chains give.  Measured (us forward / dQ / dK/dV at 1, 2, 4 waves per tile,
+// 16 causal sequences of mean 256 or 512): head_dim 64, 1,184 row tiles (4 x
+// 1,024) 94/132/170, 72/95/123, 66/96/115; 1,504: 51/74/92, 38/49/63,
+// 36/53/66; 3,792: 114/164/218, 100/149/185, 106/164/208; 5,056: 127/184/234,
+// 126/197/239, 137/213/268; head_dim 32, 2,528: 62/88/113, 45/58/71,
+// 39/55/77; 9,088 (64 x 128, no mask): 63/90/119, 64/94/131, 71/110/154;
+// head_dim 128 (one wave per SIMD), 1,264: 177/263/346, 95/138/182,
+// 106/157/185; 2,528: 185/270/346, 168/252/303, 199/300/351; 3,792:
+// 260/380/442, 269/393/450, 318/465/538.
 template <int D>
-bool f32_use_wide(int64_t grid) {
-  constexpr int64_t waves = (f32_threads<D, kF32NarrowDpt>() + kWave - 1) / kWave;
-  return f32_wide_dpt<D>() != kF32NarrowDpt && grid * waves < 1024;
+int f32m_share(int64_t blocks) {
+  const int64_t tiles = 4 * blocks;
+  constexpr int64_t kSimds = 1024;
+  if (tiles < (D >= 64 ? 1 : 2) * kSimds) return 4;
+  return tiles < (D >= 128 ? 3 : 5) * kSimds ? 2 : 1;
 }
-
-template <int D, bool C, int DPT, int KG>
-void launch_fwd_f32_as(const void* q, const void* k, const void* v, void* o, float* lse,
-                       const int32_t* cu, int batch, int heads, int kv_heads, const int64_t* st,
-                       float scale, int tmax, void* ws, int total, hipStream_t stream) {
-  const int64_t grid = (int64_t)tmax * heads * kF32Split;
-  const int hm = attn_head_major(heads, tmax);
-  hipLaunchKernelGGL((attn_fwd_f32_kernel<D, C, DPT, KG>), dim3((unsigned)grid),
-                     dim3(f32_threads<D, DPT, KG>()), 0,
-                     stream, static_cast<const float*>(q), static_cast<const float*>(k),
-                     static_cast<const float*>(v), static_cast<float*>(o), lse,
-                     fwd_item_source(ws, cu, batch, total, tmax, heads, D, hm), tmax, hm, heads,
-                     heads / kv_heads, Strides{st[0], st[1]}, Strides{st[2], st[3]},
-                     Strides{st[4], st[5]}, Strides{st[6], st[7]}, scale, total);
+template <int KG>
+dim3 f32m_grid(int64_t blocks) {  // whole groups of kXcds * KG (f32m_block)
+  return dim3((unsigned)((blocks + kXcds - 1) / kXcds * kXcds * KG));
 }
+// KERNEL for this launch's share, or, at head_dim 256, FMA_KERNEL.  A row
+// tile that sweeps its sequence `sweeps` times (dK/dV: the query heads of a
+// group) has as much the longer a chain: 16 heads on 4 K/V heads of 64, 1,264
+// row tiles, dK/dV 249 us at 4 waves per tile, 417 at 2.
+#define SCREE_LAUNCH_F32(KERNEL, FMA_KERNEL, D, C, blocks, sweeps, stream, ...)                    \
+  do {                                                                                             \
+    const int64_t blocks_ = (blocks);                                                              \
+    if constexpr (D > 128) {                                                                       \
+      hipLaunchKernelGGL((FMA_KERNEL<D, C>), dim3((unsigned)(blocks_ * kF32Split)),                \
+                         dim3(f32_threads<D>()), 0, stream, __VA_ARGS__);                          \
+    } else {                                                                                       \
+      const int share_ = f32m_share<D>(blocks_ / (sweeps));                                        \
+      if (share_ == 4)                                                                             \
+        hipLaunchKernelGGL((KERNEL<D, C, 4>), f32m_grid<4>(blocks_), dim3(kThreads), 0, stream,    \
+                           __VA_ARGS__);                                                           \
+      else if (share_ == 2)                                                                        \
+        hipLaunchKernelGGL((KERNEL<D, C, 2>), f32m_grid<2>(blocks_), dim3(kThreads), 0, stream,    \
+                           __VA_ARGS__);                                                           \
+      else                                                                                         \
+        hipLaunchKernelGGL((KERNEL<D, C, 1>), f32m_grid<1>(blocks_), dim3(kThreads), 0, stream,    \
+                           __VA_ARGS__);                                                           \
+    }                                                                                              \
+  } while (0)
 
 template <int D, bool C>
 void launch_fwd_f32(const void* q, const void* k, const void* v, void* o, float* lse,
                     const int32_t* cu, int batch, int heads, int kv_heads, const int64_t* st,
                     float scale, int tmax, void* ws, int total, hipStream_t stream) {
-  if constexpr (f32_wide_dpt<D>() != kF32NarrowDpt) {  // (head_dim 256 has no wide form)
-    if (f32_use_wide<D>((int64_t)tmax * heads * kF32Split)) {
-      launch_fwd_f32_as<D, C, f32_wide_dpt<D>(), 2>(q, k, v, o, lse, cu, batch, heads, kv_heads,
-                                                    st, scale, tmax, ws, total, stream);
-      return;
-    }
-  }
-  launch_fwd_f32_as<D, C, kF32NarrowDpt, 1>(q, k, v, o, lse, cu, batch, heads, kv_heads, st, scale,
-                                            tmax, ws, total, stream);
+  const int hm = attn_head_major(heads, tmax);
+  SCREE_LAUNCH_F32(attn_fwd_f32m_kernel, attn_fwd_f32_kernel, D, C, (int64_t)tmax * heads, 1,
+                   stream, static_cast<const float*>(q), static_cast<const float*>(k),
+                   static_cast<const float*>(v), static_cast<float*>(o), lse,
+                   fwd_item_source(ws, cu, batch, total, tmax, heads, D, hm), tmax, hm, heads,
+                   heads / kv_heads, Strides{st[0], st[1]}, Strides{st[2], st[3]},
+                   Strides{st[4], st[5]}, Strides{st[6], st[7]}, scale, total);
 }
 
 // strides: {dout, q, k, v, o, dq} x {row, head}
-template <int D, bool C, int DPT, int KG>
-void launch_bwd_dq_f32_as(const void* dout, const void* q, const void* k, const void* v,
-                          const void* o, const float* lse, void* dq, float* delta, int heads,
-                          int kv_heads, const int64_t* st, float scale, int tmax, const void* ws,
-                          int total, hipStream_t stream) {
-  const int64_t grid = (int64_t)tmax * heads * kF32Split;
-  const int hm = attn_head_major(heads, tmax);
-  hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<D, C, DPT, KG>), dim3((unsigned)grid),
-                     dim3(f32_threads<D, DPT, KG>()), 0, stream, static_cast<const float*>(dout), static_cast<const float*>(q),
-                     static_cast<const float*>(k), static_cast<const float*>(v),
-                     static_cast<const float*>(o), lse, delta, static_cast<float*>(dq),
-                     list_item_source(ws, total, tmax, hm), tmax, hm, heads, heads / kv_heads,
-                     Strides{st[0], st[1]}, Strides{st[2], st[3]}, Strides{st[4], st[5]},
-                     Strides{st[6], st[7]}, Strides{st[8], st[9]}, Strides{st[10], st[11]}, scale,
-                     total);
-}
-
 template <int D, bool C>
 void launch_bwd_dq_f32(const void* dout, const void* q, const void* k, const void* v,
                        const void* o, const float* lse, void* dq, float* delta, int heads,
                        int kv_heads, const int64_t* st, float scale, int tmax, const void* ws,
                        int total, hipStream_t stream) {
-  if constexpr (f32_wide_dpt<D>() != kF32NarrowDpt) {
-    if (f32_use_wide<D>((int64_t)tmax * heads * kF32Split)) {
-      launch_bwd_dq_f32_as<D, C, f32_wide_dpt<D>(), 2>(dout, q, k, v, o, lse, dq, delta, heads,
-                                                       kv_heads, st, scale, tmax, ws, total, stream);
-      return;
-    }
-  }
-  launch_bwd_dq_f32_as<D, C, kF32NarrowDpt, 1>(dout, q, k, v, o, lse, dq, delta, heads, kv_heads,
-                                               st, scale, tmax, ws, total, stream);
+  const int hm = attn_head_major(heads, tmax);
+  SCREE_LAUNCH_F32(attn_bwd_dq_f32m_kernel, attn_bwd_dq_f32_kernel, D, C, (int64_t)tmax * heads,
+                   1, stream, static_cast<const float*>(dout), static_cast<const float*>(q),
+                   static_cast<const float*>(k), static_cast<const float*>(v),
+                   static_cast<const float*>(o), lse, delta, static_cast<float*>(dq),
+                   list_item_source(ws, total, tmax, hm), tmax, hm, heads, heads / kv_heads,
+                   Strides{st[0], st[1]}, Strides{st[2], st[3]}, Strides{st[4], st[5]},
+                   Strides{st[6], st[7]}, Strides{st[8], st[9]}, Strides{st[10], st[11]}, scale,
+                   total);
 }
 
-// strides: {dout, q, k, v, dk, dv} x {row, head}; one workgroup per (item, K/V head)
-template <int D, bool C, int DPT, int KG>
-void launch_bwd_dkv_f32_as(const void* dout, const void* q, const void* k, const void* v,
-                           const float* lse, const float* delta, void* dk, void* dv, int heads,
-                           int kv_heads, const int64_t* st, float scale, int tmax, const void* ws,
-                           int total, hipStream_t stream) {
-  const int64_t grid = (int64_t)tmax * kv_heads * kF32Split;
-  const int hm = attn_head_major(kv_heads, tmax);
-  hipLaunchKernelGGL((attn_bwd_dkv_f32_kernel<D, C, DPT, KG>), dim3((unsigned)grid),
-                     dim3(f32_threads<D, DPT, KG>()), 0, stream, static_cast<const float*>(dout), static_cast<const float*>(q),
-                     static_cast<const float*>(k), static_cast<const float*>(v), lse, delta,
-                     static_cast<float*>(dk), static_cast<float*>(dv),
-                     list_item_source(ws, total, tmax, hm), tmax, hm, kv_heads,
-                     heads / kv_heads, Strides{st[0], st[1]}, Strides{st[2], st[3]},
-                     Strides{st[4], st[5]}, Strides{st[6], st[7]}, Strides{st[8], st[9]},
-                     Strides{st[10], st[11]}, scale, total);
-}
-
+// strides: {dout, q, k, v, dk, dv} x {row, head}; blocks are (item, K/V head) pairs
 template <int D, bool C>
 void launch_bwd_dkv_f32(const void* dout, const void* q, const void* k, const void* v,
                         const float* lse, const float* delta, void* dk, void* dv, int heads,
                         int kv_heads, const int64_t* st, float scale, int tmax, const void* ws,
                         int total, hipStream_t stream) {
-  if constexpr (f32_wide_dpt<D>() != kF32NarrowDpt) {
-    if (f32_use_wide<D>((int64_t)tmax * kv_heads * kF32Split)) {
-      // one query group at head_dim 128: two would need 1,024 threads of more
-      // than the 128 registers each that allows
-      constexpr int KG = D >= 128 ? 1 : 2;
-      launch_bwd_dkv_f32_as<D, C, f32_wide_dpt<D>(), KG>(dout, q, k, v, lse, delta, dk, dv, heads,
-                                                         kv_heads, st, scale, tmax, ws, total,
-                                                         stream);
-      return;
-    }
-  }
-  launch_bwd_dkv_f32_as<D, C, kF32NarrowDpt, 1>(dout, q, k, v, lse, delta, dk, dv, heads, kv_heads,
-                                                st, scale, tmax, ws, total, stream);
+  const int hm = attn_head_major(kv_heads, tmax);
+  SCREE_LAUNCH_F32(attn_bwd_dkv_f32m_kernel, attn_bwd_dkv_f32_kernel, D, C,
+                   (int64_t)tmax * kv_heads, heads / kv_heads, stream, static_cast<const float*>(dout),
+                   static_cast<const float*>(q), static_cast<const float*>(k),
+                   static_cast<const float*>(v), lse, delta, static_cast<float*>(dk),
+                   static_cast<float*>(dv), list_item_source(ws, total, tmax, hm), tmax, hm,
+                   kv_heads, heads / kv_heads, Strides{st[0], st[1]}, Strides{st[2], st[3]},
+                   Strides{st[4], st[5]}, Strides{st[6], st[7]}, Strides{st[8], st[9]},
+                   Strides{st[10], st[11]}, scale, total);
 }
 
 }  // namespace

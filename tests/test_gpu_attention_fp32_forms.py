@@ -1,0 +1,54 @@
+"""GPU parity of the fp32 matrix-instruction attention at the sizes where its
+forms can go wrong: sequence lengths around the 32-row tile and the 128-row
+item, with 4, 2 and 1 waves sharing a row tile (the launchers choose by the
+number of row tiles: 4 below 2,048, or 1,024 from head_dim 64 up; 2 below
+5,120, or 3,072 at head_dim 128), in both mask modes, with and without grouped
+K/V heads.  Bounds as in ``test_gpu_attention_fp32``.
+"""
+
+import pytest
+import torch
+
+from parity import cu_of, randn, say
+from test_gpu_attention_fp32 import run_fp32_case
+
+pytestmark = pytest.mark.gpu
+
+# 19 row blocks per head (ceil(868 / 128) + 12), 76 row tiles
+TILE_LENGTHS = [1, 31, 32, 33, 64, 65, 96, 127, 128, 129, 160, 2]
+
+
+@pytest.mark.parametrize("heads", [8, 32, 84])  # 608, 2,432 and 6,384 row tiles: 4, 2, 1 waves
+@pytest.mark.parametrize("dim", [16, 32, 64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fp32_waves_per_row_tile(dim, heads, causal):
+    # grouped K/V heads below 64 columns; without them the dK/dV pass takes the same form
+    run_fp32_case(TILE_LENGTHS, heads, dim, causal, seed=900 + dim,
+                  kv_heads=heads // 2 if dim < 64 else heads)
+
+
+@pytest.mark.parametrize("dim", [16, 64, 128])
+def test_fp32_single_token_any_row_stride(dim):
+    """One token whose row stride says nothing (0, as a size-1 axis may have):
+    the same output and gradients as from a contiguous tensor."""
+    import scree_amd
+    from scree_amd.kernels import varlen_attention
+
+    say(f"case: fp32 one token, row stride 0, D={dim}")
+    _, cu = cu_of([1])
+    heads = 4
+    base = [randn((1, heads, dim), torch.float32, 40 + i) for i in range(4)]
+
+    def run(ts):
+        qa, ka, va = (t.detach().requires_grad_(True) for t in ts[:3])
+        out = varlen_attention(*(scree_amd.Array(values=t, offsets=cu) for t in (qa, ka, va)),
+                               causal=True).values
+        out.backward(ts[3])
+        return [out.detach(), qa.grad, ka.grad, va.grad]
+
+    got = run([t.as_strided((1, heads, dim), (0, dim, 1)) for t in base])
+    want = run(base)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], base[2])  # the only key's value
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
