@@ -6,18 +6,22 @@
 //
 // Fast path: one wavefront per row.  Each lane keeps CHUNKS 16-byte vectors
 // of the row in registers (dim = CHUNKS * 64 lanes * 16 bytes at most), so x
-// is read from HBM exactly once; the reductions are wave-wide shuffles.
+// is read from HBM exactly once; the reductions are wave-wide shuffles.  Rows
+// of at most 128 vectors take 4 to 64 lanes each (short rows, below).
 // Generic path (dim not a multiple of one 16-byte vector, unaligned buffers,
 // or rows longer than the fast path holds): one wavefront per row looping
 // over the columns.
 //
-// Backward (norm_bwd_cols): each thread of a block owns fixed 16-byte column
-// vectors across the block's rows, so the parameter gradients accumulate in
+// Backward (norm_bwd_cols): each thread of a block (or, at up to 256 vectors
+// per row, of a team of waves in it) owns fixed 16-byte column vectors across
+// the block's rows, so the parameter gradients accumulate in
 // its fp32 registers; the row statistics are reduced across the block through
 // LDS, dx is written per row, and each block writes one partial row of
 // parameter gradients, which a column-sum kernel adds in a fixed order.  No
 // atomics: results are bit-identical from run to run.
+#include <algorithm>
 #include <initializer_list>
+#include <type_traits>
 
 #include "common.h"
 
@@ -163,6 +167,159 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
   }
 }
 
+// ------------------------------------------------------------- short rows
+// Rows of at most 256 16-byte vectors (2,048 columns in 16 bits, 1,024 in
+// fp32).  A wave-per-row or block-per-row kernel leaves most of its lanes
+// without a column there: at 128 bf16 columns 16 of a wave's 64, and 16 of the
+// 512 threads of norm_bwd_cols.  Here LPR lanes (a power of two) hold a row,
+// CH vectors each, so a wave holds 64 / LPR rows; the host picks the pair that
+// covers the row with the fewest idle lanes (short_shape).  Row sums are DPP
+// and permlane steps within the LPR lanes: no LDS, no barrier.  Bound by HBM
+// on large inputs.  Measured (us, forward RMS / LN / add, backward RMS / LN /
+// add; the wave-per-row and norm_bwd_cols kernels before):
+//   194,560 x 128 bf16  44/61/72, 246/301/462 -> 19/21/36, 32/33/38
+//   100,000 x 32 fp32   20/27/28,  88/108/206 ->  6/7/11,  12/13/14
+//   12,160 x 768 fp16    9/12/15,   25/32/40  ->  8/8/14,  18/20/20
+//   12,160 x 1,024 bf16 11/13/19,   27/31/42  -> 11/12/18, 20/22/23
+// From 129 to 256 vectors a row the backward's norm_bwd_cols takes several
+// rows per block instead (teams of waves): 12,160 x 1,536 bf16 30/35/46 ->
+// 26/29/34, x 2,048 34/39/50 -> 31/34/40.
+//
+// Sum over the two 32-lane halves, and over the two 16-lane rows of each half,
+// in every lane: the permlane swaps exchange halves (rows) of two copies, so
+// one holds the lower and the other the upper value.  (Written out: the
+// builtin folds two equal inputs into one result.)
+__device__ __forceinline__ float halves_sum(float x) {
+  float lo = x, hi = x;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+  return lo + hi;
+}
+__device__ __forceinline__ float rows_sum(float x) {
+  float lo = x, hi = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+  return lo + hi;
+}
+template <int LPR>
+__device__ __forceinline__ float group_sum(float v) {
+  static_assert(LPR >= 4 && LPR <= 64 && (LPR & (LPR - 1)) == 0, "LPR: a power of two, 4 to 64");
+  auto dpp = [](float x, auto ctrl) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                   0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  v = dpp(v, std::integral_constant<int, 0xB1>{});                             // lane ^ 1
+  v = dpp(v, std::integral_constant<int, 0x4E>{});                             // lane ^ 2
+  if constexpr (LPR >= 8) v = dpp(v, std::integral_constant<int, 0x141>{});   // across 4 (half mirror)
+  if constexpr (LPR >= 16) v = dpp(v, std::integral_constant<int, 0x140>{});  // across 8 (mirror)
+  if constexpr (LPR >= 32) v = rows_sum(v);
+  if constexpr (LPR >= 64) v = halves_sum(v);
+  return v;
+}
+// The converse: the sum of lane l of every LPR-lane group of the wave.
+template <int LPR>
+__device__ __forceinline__ float subgroups_sum(float v) {
+  auto dpp = [](float x, auto ctrl) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                   0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  if constexpr (LPR <= 4) v = dpp(v, std::integral_constant<int, 0x124>{});  // rotate by 4 in the row
+  if constexpr (LPR <= 8) v = dpp(v, std::integral_constant<int, 0x128>{});  // by 8
+  if constexpr (LPR <= 16) v = rows_sum(v);
+  if constexpr (LPR <= 32) v = halves_sum(v);
+  return v;
+}
+// Row groups a wave of the forward loads before it reduces any, in launches
+// that still give every CU two workgroups; below that one group per wave (613
+// x 192 bf16: 4.2 us with four groups, 3.4 with one; 12,160 x 768 fp16: 7.5 us
+// with two, 8.0 with one).
+template <int CH>
+constexpr int short_groups() {
+  return CH == 1 ? 4 : 2;
+}
+
+template <typename T, int LPR, int CH, int G, bool LAYER, bool RES>
+__global__ __launch_bounds__(kFwdWaves* kWave) void norm_fwd_short(
+    const T* __restrict__ x, const T* __restrict__ res, const T* __restrict__ w,
+    const T* __restrict__ b, T* __restrict__ hout, T* __restrict__ y,
+    float* __restrict__ mean_out, float* __restrict__ rstd_out, int64_t rows, int dim, float eps) {
+  constexpr int VEC = 16 / sizeof(T), RPW = kWave / LPR;
+  const int lane = threadIdx.x & (kWave - 1), l = lane % LPR;
+  const int nvec = dim / VEC;
+  // consecutive waves take consecutive row groups, a workgroup G strips of them
+  const int64_t first = ((int64_t)blockIdx.x * G * kFwdWaves + threadIdx.x / kWave) * RPW + lane / LPR;
+  uint4 v[G][CH], rv[RES ? G : 1][CH], wv[CH], bv[LAYER ? CH : 1];
+  bool own[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) own[c] = c * LPR + l < nvec;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t row = first + g * kFwdWaves * RPW;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int64_t off = row * dim + (c * LPR + l) * VEC;
+      const bool ok = own[c] && row < rows;
+      v[g][c] = ok ? ld16_nt(x + off) : make_uint4(0, 0, 0, 0);
+      if (RES) rv[g][c] = ok ? ld16_nt(res + off) : make_uint4(0, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int64_t off = (c * LPR + l) * VEC;
+    wv[c] = (w && own[c]) ? ld16(w + off) : make_uint4(0, 0, 0, 0);
+    if (LAYER) bv[c] = (b && own[c]) ? ld16(b + off) : make_uint4(0, 0, 0, 0);
+  }
+  const float fdim = (float)dim;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t row = first + g * kFwdWaves * RPW;
+    const bool live = row < rows;
+    if (RES) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        float f[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) f[e] = elem<T>(v[g][c], e) + elem<T>(rv[g][c], e);
+        v[g][c] = pack16<T>(f);
+        if (live && own[c]) st16_nt(hout + row * dim + (c * LPR + l) * VEC, v[g][c]);
+      }
+    }
+    float mu = 0.f, s = 0.f;
+    if (LAYER) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) s += elem<T>(v[g][c], e);
+      mu = group_sum<LPR>(s) / fdim;
+      s = 0.f;
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (LAYER && !own[c]) continue;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float d = LAYER ? elem<T>(v[g][c], e) - mu : elem<T>(v[g][c], e);
+        s = __builtin_fmaf(d, d, s);
+      }
+    }
+    const float rstd = 1.0f / sqrtf(group_sum<LPR>(s) / fdim + eps);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      float f[VEC];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        float t = LAYER ? (elem<T>(v[g][c], e) - mu) * rstd : elem<T>(v[g][c], e) * rstd;
+        if (w) t *= elem<T>(wv[c], e);
+        if (LAYER && b) t += elem<T>(bv[c], e);
+        f[e] = t;
+      }
+      if (live && own[c]) st16_nt(y + row * dim + (c * LPR + l) * VEC, pack16<T>(f));
+    }
+    if (live && l == 0) {
+      if (rstd_out) rstd_out[row] = rstd;
+      if (LAYER && mean_out) mean_out[row] = mu;
+    }
+  }
+}
+
 template <typename T, bool LAYER, bool RES>
 __global__ __launch_bounds__(kFwdWaves* kWave) void norm_fwd_generic(
     const T* __restrict__ x, const T* __restrict__ res, const T* __restrict__ w,
@@ -237,7 +394,7 @@ constexpr int kBwdWarps = kBwdThreads / kWave;
 // One step's rows: this thread's 16-byte vectors of x, dy (and dres) for R
 // rows, with the rows' statistics.  The kernel keeps two of these and loads
 // the next step's rows while it reduces and writes the current one.
-template <typename T, int CPT, int R, bool LAYER, bool RES>
+template <typename T, int CPT, int R, int TEAM, bool LAYER, bool RES>
 struct BwdRows {
   uint4 xv[R][CPT], gv[R][CPT], hv[RES ? R : 1][CPT];
   float rs[R], mu[R];
@@ -256,7 +413,7 @@ struct BwdRows {
       mu[r] = (LAYER && ok) ? mean_in[row] : 0.f;
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
-        const int64_t off = row * (int64_t)dim + (int64_t)(tid + k * kBwdThreads) * VEC;
+        const int64_t off = row * (int64_t)dim + (int64_t)(tid + k * TEAM) * VEC;
         xv[r][k] = (ok && own[k]) ? ld16_nt(x + off) : make_uint4(0, 0, 0, 0);
         gv[r][k] = (ok && own[k]) ? ld16_nt(dy + off) : make_uint4(0, 0, 0, 0);
         if (RES) hv[r][k] = (ok && own[k]) ? ld16_nt(dres + off) : make_uint4(0, 0, 0, 0);
@@ -273,9 +430,9 @@ struct BwdRows {
 //   LayerNorm  dx = rstd * g - rstd*b * x-hat - rstd*a,  a = mean(g), b = mean(g * x-hat)
 //   RMSNorm    dx = rstd * g - k * x,                    k = rstd^3 * mean(g * x)
 // with g = dy * w (reference varlen_layernorm.py:64-74, varlen_rmsnorm.py:58-65).
-template <typename T, int CPT, int R, bool LAYER, bool RES>
-__device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, LAYER, RES>& st,
-                                              float (&red)[2][R][2][kBwdWarps], int buf,
+template <typename T, int CPT, int R, int TEAM, bool LAYER, bool RES>
+__device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, TEAM, LAYER, RES>& st,
+                                              float (&red)[2][R][2][TEAM / kWave], int buf,
                                               const float (&wf)[CPT][16 / sizeof(T)],
                                               const bool* own,
                                               float (&aw)[CPT][16 / sizeof(T)],
@@ -330,7 +487,7 @@ __device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, LAYER, RES>& st
   for (int r = 0; r < R; ++r) {
     float t1 = 0.f, t2 = 0.f;
 #pragma unroll
-    for (int q = 0; q < kBwdWarps; ++q) {
+    for (int q = 0; q < TEAM / kWave; ++q) {
       t1 += red[buf][r][0][q];
       if (LAYER) t2 += red[buf][r][1][q];
     }
@@ -361,29 +518,32 @@ __device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, LAYER, RES>& st
         }
         if (RES) f[e] += elem<T>(st.hv[RES ? r : 0][k], e);
       }
-      st16_nt(dx + row * (int64_t)dim + (int64_t)(tid + k * kBwdThreads) * VEC, pack16<T>(f));
+      st16_nt(dx + row * (int64_t)dim + (int64_t)(tid + k * TEAM) * VEC, pack16<T>(f));
     }
   }
 }
 
 // RES: dx also receives dres (the gradient reaching the normalised input by
 // another path, e.g. the residual stream of an add + RMSNorm).
-template <typename T, int CPT, int R, bool LAYER, bool RES>
-__global__ __launch_bounds__(kBwdThreads) void norm_bwd_cols(
+template <typename T, int CPT, int R, int TW, int TEAMS, bool LAYER, bool RES>
+__global__ __launch_bounds__(TW* TEAMS* kWave) void norm_bwd_cols(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ mean_in, const float* __restrict__ rstd_in,
     const T* __restrict__ dres, T* __restrict__ dx, float* __restrict__ partial, int64_t rows,
     int dim, int nparam) {
   constexpr int VEC = 16 / sizeof(T);
-  __shared__ float red[2][R][2][kBwdWarps];
-  const int tid = threadIdx.x;
+  constexpr int TEAM = TW * kWave;
+  __shared__ float red[TEAMS][2][R][2][TW];
+  // (a team is whole waves: its index, and with it every row's address, is scalar)
+  const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / TEAM) : 0;
+  const int tid = (int)threadIdx.x - team * TEAM;
   const int nvec = dim / VEC;
 
   float wf[CPT][VEC];  // this thread's weights as fp32, ones without a weight
   bool own[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int v = tid + k * kBwdThreads;
+    const int v = tid + k * TEAM;
     own[k] = v < nvec;
     const uint4 wv = (w && own[k]) ? ld16(w + (int64_t)v * VEC) : make_uint4(0, 0, 0, 0);
 #pragma unroll
@@ -401,29 +561,220 @@ __global__ __launch_bounds__(kBwdThreads) void norm_bwd_cols(
   // Two row sets: while one step reduces and writes, the next step's rows
   // load.  Steps are S rows apart; rows past the end load as zeros and are
   // not written.
-  BwdRows<T, CPT, R, LAYER, RES> A, B;
+  BwdRows<T, CPT, R, TEAM, LAYER, RES> A, B;
   const float inv_dim = 1.0f / (float)dim;
-  const int64_t S = (int64_t)gridDim.x * R;
-  const int64_t first = (int64_t)blockIdx.x * R;
-  if (first < rows) A.load(x, dy, dres, mean_in, rstd_in, own, first, rows, dim, tid);
-  for (int64_t rb = first; rb < rows; rb += 2 * S) {
-    if (rb + S < rows) B.load(x, dy, dres, mean_in, rstd_in, own, rb + S, rows, dim, tid);
-    norm_bwd_step<T, CPT, R, LAYER, RES>(A, red, 0, wf, own, aw, ab, dx, rb, rows, dim, inv_dim, tid);
-    if (rb + S >= rows) break;
-    if (rb + 2 * S < rows) A.load(x, dy, dres, mean_in, rstd_in, own, rb + 2 * S, rows, dim, tid);
-    norm_bwd_step<T, CPT, R, LAYER, RES>(B, red, 1, wf, own, aw, ab, dx, rb + S, rows, dim, inv_dim, tid);
+  // (with several teams every one runs the block's count of steps: they share
+  // the steps' barriers; rows past the end load as zeros)
+  const int64_t S = (int64_t)gridDim.x * TEAMS * R;
+  const int64_t lead = (int64_t)blockIdx.x * TEAMS * R;  // the block's first row
+  const int64_t first = lead + team * R, lag = first - lead;
+  if (lead < rows) A.load(x, dy, dres, mean_in, rstd_in, own, first, rows, dim, tid);
+  for (int64_t rb = first; rb - lag < rows; rb += 2 * S) {
+    if (rb - lag + S < rows) B.load(x, dy, dres, mean_in, rstd_in, own, rb + S, rows, dim, tid);
+    norm_bwd_step<T, CPT, R, TEAM, LAYER, RES>(A, red[team], 0, wf, own, aw, ab, dx, rb, rows, dim, inv_dim, tid);
+    if (rb - lag + S >= rows) break;
+    if (rb - lag + 2 * S < rows) A.load(x, dy, dres, mean_in, rstd_in, own, rb + 2 * S, rows, dim, tid);
+    norm_bwd_step<T, CPT, R, TEAM, LAYER, RES>(B, red[team], 1, wf, own, aw, ab, dx, rb + S, rows, dim, inv_dim, tid);
   }
-  for (int p = 0; p < nparam; ++p) {
+  __shared__ __align__(16) float tsum[TEAMS > 1 ? TEAMS - 1 : 1][TEAMS > 1 ? CPT * TEAM * VEC : 1];
+  auto write = [&](int p, auto& acc) {
     float* out = partial + ((int64_t)blockIdx.x * nparam + p) * dim;
+    if constexpr (TEAMS > 1) {  // the other teams' sums, added in team order
+      __syncthreads();
+      if (team > 0) {
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) tsum[team - 1][(tid + k * TEAM) * VEC + e] = acc[k][e];
+      }
+      __syncthreads();
+      if (team > 0) return;
+#pragma unroll
+      for (int t = 0; t < TEAMS - 1; ++t)
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) acc[k][e] += tsum[t][(tid + k * TEAM) * VEC + e];
+    }
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       if (!own[k]) continue;
-      float* o = out + (int64_t)(tid + k * kBwdThreads) * VEC;
+      float* o = out + (int64_t)(tid + k * TEAM) * VEC;
 #pragma unroll
-      for (int e = 0; e < VEC; e += 4) {
-        const float* src = p == 0 ? &aw[k][e] : &ab[LAYER ? k : 0][e];
-        *reinterpret_cast<float4*>(o + e) = make_float4(src[0], src[1], src[2], src[3]);
+      for (int e = 0; e < VEC; e += 4)
+        *reinterpret_cast<float4*>(o + e) = make_float4(acc[k][e], acc[k][e + 1], acc[k][e + 2], acc[k][e + 3]);
+    }
+  };
+  if (nparam > 0) write(0, aw);
+  if constexpr (LAYER) {
+    if (nparam > 1) write(1, ab);
+  }
+}
+
+// Short rows (see norm_fwd_short).  A lane keeps its columns' parameter sums in
+// registers over every row it takes; at the end the wave's row groups are
+// summed by lane exchanges and the block's waves through LDS, in a fixed
+// order, into the block's partial row.  Blocks take interleaved row groups as
+// in norm_bwd_cols; the next group loads during the current one where both fit
+// 128 registers (CH == 1), else four waves per SIMD cover the loads.
+template <typename T, int LPR, int CH, bool LAYER, bool RES>
+struct ShortRows {
+  uint4 xv[CH], gv[CH], hv[CH];
+  float rs, mu;
+  __device__ __forceinline__ void load(const T* __restrict__ x, const T* __restrict__ dy,
+                                       const T* __restrict__ dres,
+                                       const float* __restrict__ mean_in,
+                                       const float* __restrict__ rstd_in, const bool (&own)[CH],
+                                       int64_t row, int64_t rows, int dim, int l) {
+    constexpr int VEC = 16 / sizeof(T);
+    const bool ok = row < rows;
+    rs = ok ? rstd_in[row] : 0.f;
+    mu = (LAYER && ok) ? mean_in[row] : 0.f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int64_t off = row * dim + (c * LPR + l) * VEC;
+      xv[c] = (ok && own[c]) ? ld16_nt(x + off) : make_uint4(0, 0, 0, 0);
+      gv[c] = (ok && own[c]) ? ld16_nt(dy + off) : make_uint4(0, 0, 0, 0);
+      if (RES) hv[c] = (ok && own[c]) ? ld16_nt(dres + off) : make_uint4(0, 0, 0, 0);
+    }
+  }
+};
+// An empty asm over a packed vector: the compiler unpacks it again after it
+// instead of holding the converted floats.
+__device__ __forceinline__ void repack(uint4& v) {
+  asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
+}
+// One step's rows; arithmetic per row as in norm_bwd_step.
+template <typename T, int LPR, int CH, bool LAYER, bool RES>
+__device__ __forceinline__ void norm_bwd_short_step(
+    ShortRows<T, LPR, CH, LAYER, RES>& st, uint4 (&wv)[CH], bool has_w, const bool (&own)[CH],
+    float (&aw)[CH][16 / sizeof(T)], float (&ab)[LAYER ? CH : 1][16 / sizeof(T)],
+    T* __restrict__ dx, int64_t row, int64_t rows, int dim, float inv_dim, int l) {
+  constexpr int VEC = 16 / sizeof(T);
+  const float rr = st.rs, nmr = -st.mu * rr;
+  float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    repack(wv[c]);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float xx = elem<T>(st.xv[c], e);
+      const float d = elem<T>(st.gv[c], e);
+      const float g = has_w ? d * elem<T>(wv[c], e) : d;
+      if (LAYER) {
+        s1 += g;
+        s2 = fmaf(g, fmaf(xx, rr, nmr), s2);
+      } else {
+        s1 = fmaf(xx, g, s1);
       }
+    }
+  }
+  s1 = group_sum<LPR>(s1);
+  if (LAYER) s2 = group_sum<LPR>(s2);
+  const float c1 = -rr * (s1 * inv_dim);
+  const float c2 = LAYER ? -rr * (s2 * inv_dim) : -(rr * rr * rr) * (s1 * inv_dim);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    repack(st.xv[c]);
+    repack(st.gv[c]);
+    repack(wv[c]);
+    float f[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float xx = elem<T>(st.xv[c], e);
+      const float d = elem<T>(st.gv[c], e);
+      const float g = has_w ? d * elem<T>(wv[c], e) : d;
+      if (LAYER) {
+        const float xh = fmaf(xx, rr, nmr);
+        f[e] = fmaf(rr, g, fmaf(c2, xh, c1));
+        aw[c][e] = fmaf(d, xh, aw[c][e]);
+        ab[LAYER ? c : 0][e] += d;
+      } else {
+        f[e] = fmaf(rr, g, c2 * xx);
+        aw[c][e] = fmaf(d * rr, xx, aw[c][e]);
+      }
+      if (RES) f[e] += elem<T>(st.hv[c], e);
+    }
+    if (row < rows && own[c]) st16_nt(dx + row * dim + (c * LPR + l) * VEC, pack16<T>(f));
+  }
+}
+template <typename T, int LPR, int CH, bool LAYER, bool RES>
+__global__ __launch_bounds__(kBwdThreads, 4) void norm_bwd_short(
+    const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
+    const float* __restrict__ mean_in, const float* __restrict__ rstd_in,
+    const T* __restrict__ dres, T* __restrict__ dx, float* __restrict__ partial, int64_t rows,
+    int dim, int nparam) {
+  constexpr int VEC = 16 / sizeof(T), RPW = kWave / LPR;
+  constexpr int RPB = kBwdWarps * RPW;  // rows of the block per step
+  __shared__ __align__(16) float sums[kBwdWarps][LPR * CH * VEC];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, l = lane % LPR;
+  const int nvec = dim / VEC;
+  bool own[CH];
+  uint4 wv[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    own[c] = c * LPR + l < nvec;
+    wv[c] = (w && own[c]) ? ld16(w + (c * LPR + l) * VEC) : make_uint4(0, 0, 0, 0);
+  }
+  float aw[CH][VEC], ab[LAYER ? CH : 1][VEC];
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      aw[c][e] = 0.f;
+      ab[LAYER ? c : 0][e] = 0.f;
+    }
+  const float inv_dim = 1.0f / (float)dim;
+  const int64_t S = (int64_t)gridDim.x * RPB;
+  int64_t row = (int64_t)blockIdx.x * RPB + wave * RPW + lane / LPR;
+  ShortRows<T, LPR, CH, LAYER, RES> A;
+  auto load = [&](ShortRows<T, LPR, CH, LAYER, RES>& st, int64_t r) {
+    st.load(x, dy, dres, mean_in, rstd_in, own, r, rows, dim, l);
+  };
+  auto step = [&](ShortRows<T, LPR, CH, LAYER, RES>& st, int64_t r) {
+    norm_bwd_short_step<T, LPR, CH, LAYER, RES>(st, wv, w != nullptr, own, aw, ab, dx, r, rows, dim,
+                                                inv_dim, l);
+  };
+  // (the loops' condition is uniform over the wave: its first row)
+  if constexpr (CH == 1) {
+    ShortRows<T, LPR, CH, LAYER, RES> B;
+    load(A, row);
+    for (; row - lane / LPR < rows; row += 2 * S) {
+      load(B, row + S);
+      step(A, row);
+      load(A, row + 2 * S);
+      step(B, row + S);
+    }
+  } else {
+#pragma unroll 1
+    for (; row - lane / LPR < rows; row += S) {
+      load(A, row);
+      step(A, row);
+    }
+  }
+  // (one call per array: a choice between them by p would keep both in memory)
+  auto write = [&](int p, const auto& acc) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float t = subgroups_sum<LPR>(acc[c][e]);
+        if (lane < LPR) sums[wave][(c * LPR + l) * VEC + e] = t;
+      }
+    __syncthreads();
+    float* out = partial + ((int64_t)blockIdx.x * nparam + p) * dim;
+    for (int i = threadIdx.x; i < dim; i += kBwdThreads) {
+      float t = sums[0][i];
+#pragma unroll
+      for (int q = 1; q < kBwdWarps; ++q) t += sums[q][i];
+      out[i] = t;
+    }
+  };
+  if (nparam > 0) write(0, aw);
+  if constexpr (LAYER) {
+    if (nparam > 1) {
+      __syncthreads();
+      write(1, ab);
     }
   }
 }
@@ -614,6 +965,28 @@ bool bwd_fast_path_ok(int64_t dim, std::initializer_list<const void*> ptrs) {
   return true;
 }
 
+// Lanes per row and vectors per lane of the short-row kernels: the pair that
+// covers nvec vectors with the fewest idle lanes, {0, 0} past their range.
+struct ShortShape {
+  int lpr, ch;
+};
+inline ShortShape short_shape(int64_t nvec, bool thirds) {
+  static const ShortShape kShapes[] = {{4, 1},  {8, 1},  {16, 1}, {32, 1},
+                                       {16, 3}, {64, 1}, {32, 3}, {64, 2}};  // by size
+  for (const ShortShape& s : kShapes)
+    if (nvec <= s.lpr * s.ch && (thirds || s.ch != 3)) return s;
+  return ShortShape{0, 0};
+}
+#define SCREE_SHORT_CASES(CASE) \
+  CASE(4, 1)                    \
+  CASE(8, 1)                    \
+  CASE(16, 1)                   \
+  CASE(32, 1)                   \
+  CASE(16, 3)                   \
+  CASE(64, 1)                   \
+  CASE(32, 3)                   \
+  CASE(64, 2)
+
 // res / h non-null (RMSNorm only): normalise h = x + res and write h too.
 template <typename T, bool LAYER, bool RES>
 void launch_fwd_k(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* yp, float* mean,
@@ -622,6 +995,25 @@ void launch_fwd_k(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* 
   const dim3 block(kFwdWaves * kWave);
   const int d = (int)dim;
   if (fast_path_ok<T>(dim, {xp, rp, wp, bp, hp, yp})) {
+    const ShortShape sh = short_shape(dim / (16 / (int64_t)sizeof(T)), true);
+    if (sh.ch) {
+#define SCREE_FWD_SHORT_G(L, C, G)                                                                 \
+  hipLaunchKernelGGL((norm_fwd_short<T, L, C, G, LAYER, RES>),                                     \
+                     dim3((unsigned)((rows + per * G - 1) / (per * G))), block, 0, stream, xp, rp, \
+                     wp, bp, hp, yp, mean, rstd, rows, d, eps)
+#define SCREE_FWD_SHORT(L, C)                                                                      \
+  if (sh.lpr == L && sh.ch == C) {                                                                 \
+    constexpr int64_t per = (int64_t)kFwdWaves * (kWave / L);                                      \
+    if (rows >= per * short_groups<C>() * 512)                                                     \
+      SCREE_FWD_SHORT_G(L, C, short_groups<C>());                                                  \
+    else                                                                                           \
+      SCREE_FWD_SHORT_G(L, C, 1);                                                                  \
+    return;                                                                                        \
+  }
+      SCREE_SHORT_CASES(SCREE_FWD_SHORT)
+#undef SCREE_FWD_SHORT
+#undef SCREE_FWD_SHORT_G
+    }
     constexpr int W = fwd_waves<LAYER>();
     const dim3 vgrid((unsigned)((rows + W - 1) / W)), vblock(W * kWave);
     const int chunks = chunks_for((int)(dim / (16 / sizeof(T))));
@@ -631,8 +1023,6 @@ void launch_fwd_k(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* 
                        hp, yp, mean, rstd, rows, d, eps);                                      \
     break;
     switch (chunks) {
-      SCREE_FWD_CASE(1)
-      SCREE_FWD_CASE(2)
       SCREE_FWD_CASE(4)
       SCREE_FWD_CASE(8)
       SCREE_FWD_CASE(16)
@@ -666,9 +1056,10 @@ int launch_fwd(const void* x, const void* res, const void* w, const void* b, voi
   return check_launch(LAYER ? "scree_layernorm_fwd" : "scree_rmsnorm_fwd");
 }
 
-// dres non-null (RMSNorm only): dx also receives dres.
+// dres non-null (RMSNorm only): dx also receives dres.  Returns the number of
+// partial rows written, at most `nparts`.
 template <typename T, bool LAYER, bool RES>
-void launch_bwd_k(const T* dyp, const T* xp, const T* wp, const float* mean, const float* rstd,
+int launch_bwd_k(const T* dyp, const T* xp, const T* wp, const float* mean, const float* rstd,
                   const T* dresp, T* dxp, float* partial, bool want_params, int nparts,
                   int64_t rows, int64_t dim, hipStream_t stream) {
   const int d = (int)dim;
@@ -678,18 +1069,39 @@ void launch_bwd_k(const T* dyp, const T* xp, const T* wp, const float* mean, con
     const int cpt = (nvec + kBwdThreads - 1) / kBwdThreads;  // 1 or 2
     const dim3 grid((unsigned)nparts), block(kBwdThreads);
     const int np = want_params ? nparam : 0;
+    // (three vectors per lane with two sums each would spill)
+    const ShortShape sh = short_shape(nvec, !LAYER);
+    if (sh.ch) {
+#define SCREE_BWD_SHORT(L, C)                                                                       \
+  if (sh.lpr == L && sh.ch == C) {                                                                  \
+    constexpr int64_t per = (int64_t)kBwdWarps * (kWave / L);          \
+    nparts = (int)std::min<int64_t>(nparts, std::max<int64_t>(1, (rows + per - 1) / per));          \
+    hipLaunchKernelGGL((norm_bwd_short<T, L, C, LAYER, RES>), dim3((unsigned)nparts), block, 0,     \
+                       stream, dyp, xp, wp, mean, rstd, dresp, dxp, partial, rows, d, np);          \
+    return nparts;                                                                                  \
+  }
+      SCREE_SHORT_CASES(SCREE_BWD_SHORT)
+#undef SCREE_BWD_SHORT
+    }
     // rows per step: two steps' rows (double-buffered) fit 4 waves per SIMD
     // (LN keeps two sums per row; the residual gradient is one more vector).
     // At one vector per thread 2 rows per step measured best for all three
     // (RMSNorm at config 2: R = 1, 2, 3, 4 -> 90.8, 87.3, 89.1, 90.5 us).
     constexpr int R1 = 2;
     constexpr int R2 = (LAYER || RES) ? 1 : 2;
-    if (cpt == 1)
-      hipLaunchKernelGGL((norm_bwd_cols<T, 1, R1, LAYER, RES>), grid, block, 0, stream, dyp, xp, wp,
-                         mean, rstd, dresp, dxp, partial, rows, d, np);
+#define SCREE_BWD_COLS(CPT, R, TW, TEAMS)                                                          \
+  hipLaunchKernelGGL((norm_bwd_cols<T, CPT, R, TW, TEAMS, LAYER, RES>), grid,                      \
+                     dim3(TW * TEAMS * kWave), 0, stream, dyp, xp, wp, mean, rstd, dresp, dxp,     \
+                     partial, rows, d, np)
+    if (nvec <= 3 * kWave)
+      SCREE_BWD_COLS(1, R1, 3, 2);
+    else if (nvec <= 4 * kWave)
+      SCREE_BWD_COLS(1, R1, 4, 2);
+    else if (cpt == 1)
+      SCREE_BWD_COLS(1, R1, kBwdWarps, 1);
     else
-      hipLaunchKernelGGL((norm_bwd_cols<T, 2, R2, LAYER, RES>), grid, block, 0, stream, dyp, xp, wp,
-                         mean, rstd, dresp, dxp, partial, rows, d, np);
+      SCREE_BWD_COLS(2, R2, kBwdWarps, 1);
+#undef SCREE_BWD_COLS
   } else {
     const dim3 grid((unsigned)((rows + kFwdWaves - 1) / kFwdWaves)), block(kFwdWaves * kWave);
     if (rows > 0)
@@ -701,6 +1113,7 @@ void launch_bwd_k(const T* dyp, const T* xp, const T* wp, const float* mean, con
                          mean, rstd, partial, rows, d, nparam);
     }
   }
+  return nparts;
 }
 
 template <typename T, bool LAYER>
@@ -715,20 +1128,20 @@ int launch_bwd(const void* dy, const void* x, const void* w, const float* mean, 
   const int d = (int)dim;
   const int nparam = LAYER ? 2 : 1;
   const bool want_params = (dw != nullptr) || (db != nullptr);
-  const int nparts = nparts_for(rows);
+  int nparts = nparts_for(rows);
   float* partial = static_cast<float*>(workspace);
   const char* fn = LAYER ? "scree_layernorm_bwd" : (dres ? "scree_add_rmsnorm_bwd" : "scree_rmsnorm_bwd");
   bool done = false;
   if constexpr (!LAYER) {
     if (dres) {
-      launch_bwd_k<T, false, true>(dyp, xp, wp, mean, rstd, dresp, dxp, partial, want_params,
-                                   nparts, rows, dim, stream);
+      nparts = launch_bwd_k<T, false, true>(dyp, xp, wp, mean, rstd, dresp, dxp, partial,
+                                            want_params, nparts, rows, dim, stream);
       done = true;
     }
   }
   if (!done)
-    launch_bwd_k<T, LAYER, false>(dyp, xp, wp, mean, rstd, nullptr, dxp, partial, want_params,
-                                  nparts, rows, dim, stream);
+    nparts = launch_bwd_k<T, LAYER, false>(dyp, xp, wp, mean, rstd, nullptr, dxp, partial,
+                                           want_params, nparts, rows, dim, stream);
   int rc = check_launch(fn);
   if (rc != SCREE_OK || !want_params) return rc;
   if (dim % 4 == 0) {
