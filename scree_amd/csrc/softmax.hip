@@ -7,20 +7,23 @@
 // / numpy per slice); it has no GPU kernel.
 //
 // Layout: x, y contiguous (total_tokens, features).  One workgroup per
-// (sequence, column chunk): its 256 threads (512 in the backward) are `ct`
+// (sequence, column chunk): its 512 threads are `ct`
 // column lanes (each owning VEC adjacent columns, one 16-byte vector when the
 // row allows it) times `threads / ct` row lanes that stride over the
 // sequence's rows.  Forward pass 1 finds each column's (max, sum of
-// exponentials); the row lanes merge through LDS; pass 2 writes the
-// normalised values with streaming stores.  Each thread keeps its first
-// kSmCache rows in registers as loaded, takes their max and then their sum,
-// and writes them in pass 2 from there, so a sequence of at most
-// kSmCache * (row lanes) rows reads x once.  Rows past that (long
-// sequences) are streamed first with an online (max, sum), one exp per
-// element, merged into the held rows' result, and re-read in pass 2 (usually
-// from the L2 / MALL).  The backward holds y and dy the same way when the
-// whole sequence fits, else streams every row twice.  Row lanes merge by a
-// fixed tree: results are deterministic.
+// exponentials); pass 2 writes the normalised values with streaming stores.
+// Each thread keeps its first kSmCache rows in registers as loaded and writes
+// them in pass 2 from there, so a sequence of at most kSmCache * (row lanes)
+// rows reads x once.  Rows past that (long sequences) are streamed first with
+// an online (max, sum), one exp per element, merged into the held rows'
+// result, and re-read in pass 2 (usually from the L2 / MALL).  The backward
+// holds y and dy the same way when the whole sequence fits, else streams
+// every row twice.  A wave's row lanes merge by lane exchanges (the wave's
+// maximum first, the exponentials against it), the waves through LDS with one
+// thread per column, in wave order: two barriers, deterministic.  A tree over
+// all row lanes in LDS (six or more barriers and 32 KB) ran the forward 82 us
+// at 19,758 x 4,096 bf16 against 79, 29 against 26 at 96 sequences of mean
+// 32, 7.2 against 5.9 at 986 x 128.
 // Statistics are fp32 for every input dtype; y has x's dtype.
 
 #include <type_traits>
@@ -114,9 +117,55 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
   return r;
 }
 
-// Merge the partial (max, sum) of another row lane into (m, l).  A lane that
-// has seen only -inf and NaN keeps m = -inf with a NaN sum: l * 0 carries it
-// (0 * 0 = 0 otherwise), and two +inf maxima give exp(inf - inf) = NaN.
+// Combine (op) the row lanes of each column within a wave: lanes l, l + ct,
+// l + 2 ct, ... hold the same columns (ct column lanes, a power of two).  DPP
+// and permlane steps, no LDS; complete in lanes < ct (the rotations leave the
+// other lanes the same terms in another order).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+}
+template <int VEC, typename Op>
+__device__ __forceinline__ void wave_columns(float (&v)[VEC], int ct, Op op) {
+  if (ct <= 1) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] = op(v[e], dpp_f<0xB1>(v[e]));  // lane ^ 1
+  }
+  if (ct <= 2) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] = op(v[e], dpp_f<0x4E>(v[e]));  // lane ^ 2
+  }
+  if (ct <= 4) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] = op(v[e], dpp_f<0x124>(v[e]));  // rotate by 4 in the row of 16
+  }
+  if (ct <= 8) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] = op(v[e], dpp_f<0x128>(v[e]));  // by 8
+  }
+  // exchanging rows (halves) of two copies leaves one with the lower and the
+  // other with the upper value (written out: the builtin folds equal inputs)
+  if (ct <= 16) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      float lo = v[e], hi = v[e];
+      asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+      v[e] = op(lo, hi);
+    }
+  }
+  if (ct <= 32) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      float lo = v[e], hi = v[e];
+      asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+      v[e] = op(lo, hi);
+    }
+  }
+}
+
+// Merge the partial (max, sum) of other rows into (m, l).  A partial that has
+// seen only -inf and NaN has m = -inf with a NaN sum: l * 0 carries it (0 * 0
+// = 0 otherwise), and two +inf maxima give exp(inf - inf) = NaN.
 __device__ __forceinline__ void sm_merge(float& m, float& l, float m2, float l2) {
   const float hi = fmaxf(m, m2);
   const float a = m == -__builtin_inff() ? l * 0.f : l * __builtin_amdgcn_exp2f((m - hi) * kLog2eSm);
@@ -139,12 +188,17 @@ __device__ __forceinline__ int sm_block(bool half_lines) {
 }
 
 template <typename T, int VEC>
-__global__ __launch_bounds__(kSmThreadsFwd) void varlen_softmax_kernel(
+__global__ __launch_bounds__(kSmThreadsFwd, 6) void varlen_softmax_kernel(
     const T* __restrict__ x, T* __restrict__ y, const int32_t* __restrict__ cu, int64_t total,
     int64_t features, int ct, int chunks) {
   constexpr int kSmThreads = kSmThreadsFwd;
-  __shared__ float s_m[kSmThreads * VEC];
-  __shared__ float s_l[kSmThreads * VEC];
+  // [wave maxima | wave sums], (kSmThreads / 64) x ct x VEC each, then the parked
+  // (max, sum) of each thread's streamed rows
+  extern __shared__ __align__(16) float sm_lds[];
+  float* red_m = sm_lds;
+  float* red_l = red_m + kSmThreads / 64 * ct * VEC;
+  float* s_m = red_l + kSmThreads / 64 * ct * VEC;
+  float* s_l = s_m + kSmThreads * VEC;
   const int bsel = sm_block(ct * VEC * (int)sizeof(T) < 128);
   const int seq = bsel / chunks, chunk = bsel - seq * chunks;
   // offsets are clamped to [0, total]: malformed input cannot index outside x
@@ -216,13 +270,24 @@ __global__ __launch_bounds__(kSmThreadsFwd) void varlen_softmax_kernel(
 #pragma unroll
       for (int e = 0; e < VEC; ++e) m[e] = max3f(m[e], a[e], b[e]);
     }
-    // The sum against mr = m, or 0 where m = -inf (every held value -inf or
-    // NaN, as v_max3 skips NaN): -inf then adds exp2(-inf) = 0 and a NaN adds
-    // NaN, as in the two-pass formula, where a guard on m = -inf would drop
-    // the NaN.
-    float mr[VEC];
+    if (excess) {
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) mr[e] = m[e] == -__builtin_inff() ? 0.f : m[e];
+      for (int e = 0; e < VEC; ++e) m[e] = fmaxf(m[e], s_m[threadIdx.x * VEC + e]);
+    }
+  }
+  // Row lanes of a wave: their maximum first, then each lane's sum of
+  // exponentials against it, then the wave's sum, by lane exchanges.
+  wave_columns<VEC>(m, ct, [](float a, float b) { return fmaxf(a, b); });
+  // complete in the wave's first ct lanes (fmaxf in any order is exact, so in all of them)
+  //
+  // The sums are against mr = m, or 0 where m = -inf (every value of the
+  // wave's rows -inf or NaN, as the maxima skip NaN): -inf then adds exp2(-inf)
+  // = 0 and a NaN adds NaN, as in the two-pass formula, where a guard on m =
+  // -inf would drop the NaN.
+  float mr[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) mr[e] = m[e] == -__builtin_inff() ? 0.f : m[e];
+  if (active) {
 #pragma unroll
     for (int i = 0; i < kSmCache; ++i) {
       if (i >= nr) continue;
@@ -231,46 +296,41 @@ __global__ __launch_bounds__(kSmThreadsFwd) void varlen_softmax_kernel(
 #pragma unroll
       for (int e = 0; e < VEC; ++e) l[e] += __builtin_amdgcn_exp2f((v[e] - mr[e]) * kLog2eSm);
     }
-    if (excess) {  // fold in the streamed rows' (max, sum)
-#pragma unroll
-      for (int e = 0; e < VEC; ++e)
-        sm_merge(m[e], l[e], s_m[threadIdx.x * VEC + e], s_l[threadIdx.x * VEC + e]);
-    }
-  }
-  // merge the row lanes of each column: a tree over the (power-of-two) row
-  // lanes in LDS, log2(rs) steps in a fixed order (deterministic)
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) {
-    s_m[threadIdx.x * VEC + e] = m[e];
-    s_l[threadIdx.x * VEC + e] = l[e];
-  }
-  for (int h = rs >> 1; h >= 1; h >>= 1) {
-    __syncthreads();
-    if (tr < h) {
+    if (excess) {  // the streamed rows' sum, rescaled (0 * NaN carries a NaN held with m = -inf)
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        const int o = ((tr + h) * ct + tc) * VEC + e;
-        sm_merge(m[e], l[e], s_m[o], s_l[o]);
-        s_m[threadIdx.x * VEC + e] = m[e];
-        s_l[threadIdx.x * VEC + e] = l[e];
+        const float em = s_m[threadIdx.x * VEC + e], el = s_l[threadIdx.x * VEC + e];
+        l[e] += el * (em == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((em - mr[e]) * kLog2eSm));
       }
     }
   }
-  __syncthreads();
-  if (tr == 0) {
+  wave_columns<VEC>(l, ct, [](float a, float b) { return a + b; });
+  // The waves' (max, sum) meet in LDS: one thread per column merges them in
+  // wave order (two barriers in all, whatever the number of row lanes).
+  constexpr int WAVES = kSmThreads / 64;
+  const int cols = ct * VEC;
+  if ((threadIdx.x & 63) < ct) {
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      s_m[tc * VEC + e] = m[e];
-      s_l[tc * VEC + e] = 1.0f / l[e];
+      red_m[(threadIdx.x / 64) * cols + tc * VEC + e] = m[e];
+      red_l[(threadIdx.x / 64) * cols + tc * VEC + e] = l[e];
     }
   }
   __syncthreads();
+  if ((int)threadIdx.x < cols) {
+    float mm = red_m[threadIdx.x], ll = red_l[threadIdx.x];
+#pragma unroll
+    for (int q = 1; q < WAVES; ++q) sm_merge(mm, ll, red_m[q * cols + threadIdx.x], red_l[q * cols + threadIdx.x]);
+    red_m[threadIdx.x] = mm;
+    red_l[threadIdx.x] = 1.0f / ll;
+  }
+  __syncthreads();
   if (!active) return;
-  float mm[VEC], inv[VEC];
+  float inv[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
-    mm[e] = s_m[tc * VEC + e];
-    inv[e] = s_l[tc * VEC + e];
+    m[e] = red_m[tc * VEC + e];
+    inv[e] = red_l[tc * VEC + e];
   }
 #pragma unroll
   for (int i = 0; i < kSmCache; ++i) {
@@ -278,7 +338,7 @@ __global__ __launch_bounds__(kSmThreadsFwd) void varlen_softmax_kernel(
     float v[VEC];
     held[i].get(v);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) v[e] = __builtin_amdgcn_exp2f((v[e] - mm[e]) * kLog2eSm) * inv[e];
+    for (int e = 0; e < VEC; ++e) v[e] = __builtin_amdgcn_exp2f((v[e] - m[e]) * kLog2eSm) * inv[e];
     Vec<T, VEC>::store(y + (start + tr + (int64_t)i * rs) * features + col, v);
   }
   for (int64_t r = start + held_rows + tr; r < end; r += kUnroll * rs) {
@@ -292,7 +352,7 @@ __global__ __launch_bounds__(kSmThreadsFwd) void varlen_softmax_kernel(
       float f[VEC];
       v[u].get(f);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) f[e] = __builtin_amdgcn_exp2f((f[e] - mm[e]) * kLog2eSm) * inv[e];
+      for (int e = 0; e < VEC; ++e) f[e] = __builtin_amdgcn_exp2f((f[e] - m[e]) * kLog2eSm) * inv[e];
       Vec<T, VEC>::store(y + (r + u * rs) * features + col, f);
     }
   }
@@ -305,7 +365,7 @@ template <typename T, int VEC>
 __global__ __launch_bounds__(kSmThreadsBwd) void varlen_softmax_bwd_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx,
     const int32_t* __restrict__ cu, int64_t total, int64_t features, int ct, int chunks) {
-  __shared__ float s_s[kSmThreadsBwd * VEC];
+  extern __shared__ __align__(16) float sm_lds[];  // wave sums, kSmThreadsBwd / 64 x ct x VEC
   const int bsel = sm_block(ct * VEC * (int)sizeof(T) < 128);
   const int seq = bsel / chunks, chunk = bsel - seq * chunks;
   const int64_t start = min<int64_t>(max<int64_t>(cu[seq], 0), total);
@@ -360,28 +420,25 @@ __global__ __launch_bounds__(kSmThreadsBwd) void varlen_softmax_bwd_kernel(
       }
     }
   }
-  // sum the row lanes of each column: tree over the row lanes (fixed order)
+  // the row lanes of each column: a wave's by lane exchanges, the waves' by one
+  // thread per column in wave order
+  wave_columns<VEC>(acc, ct, [](float a, float b) { return a + b; });
+  const int cols = ct * VEC;
+  if ((threadIdx.x & 63) < ct) {
 #pragma unroll
-  for (int e = 0; e < VEC; ++e) s_s[threadIdx.x * VEC + e] = acc[e];
-  for (int h = rs >> 1; h >= 1; h >>= 1) {
-    __syncthreads();
-    if (tr < h) {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        acc[e] += s_s[((tr + h) * ct + tc) * VEC + e];
-        s_s[threadIdx.x * VEC + e] = acc[e];
-      }
-    }
+    for (int e = 0; e < VEC; ++e) sm_lds[(threadIdx.x / 64) * cols + tc * VEC + e] = acc[e];
   }
   __syncthreads();
-  if (tr == 0) {
+  if ((int)threadIdx.x < cols) {
+    float t = sm_lds[threadIdx.x];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) s_s[tc * VEC + e] = acc[e];
+    for (int q = 1; q < kSmThreadsBwd / 64; ++q) t += sm_lds[q * cols + threadIdx.x];
+    sm_lds[threadIdx.x] = t;
   }
   __syncthreads();
   if (!active) return;
 #pragma unroll
-  for (int e = 0; e < VEC; ++e) acc[e] = s_s[tc * VEC + e];
+  for (int e = 0; e < VEC; ++e) acc[e] = sm_lds[tc * VEC + e];
   if (cached) {
 #pragma unroll
     for (int i = 0; i < kSmCacheBwd; ++i) {
@@ -435,15 +492,30 @@ SmShape sm_shape(int64_t features, bool aligned, int batch, int64_t total, int t
   // Fewer column lanes -> more chunks, more workgroups, and more row lanes,
   // i.e. longer sequences held in registers: narrow until the grid is large
   // and cache_rows rows per row lane cover twice the mean sequence length, to
-  // min_ct lanes at least.  The forward goes down to 4 (64-byte row
-  // segments, half-line chunks paired on one XCD by sm_block); the backward
-  // keeps >= 8 x 16 bytes contiguous.
+  // min_ct lanes at least (8: whole 128-byte lines).
   const int64_t cover = 2 * ((total + batch - 1) / batch);
   while (sh.ct > min_ct && ((int64_t)batch * ((units + sh.ct - 1) / sh.ct) < kSmMinBlocks ||
                        (int64_t)cache_rows * (threads / sh.ct) < cover))
     sh.ct >>= 1;
+  // A grid short of the CUs narrows further, into parts of a cache line (which
+  // several L2s then fetch): a few long sequences of few columns are bound by
+  // each workgroup's chain of rows.  Half lines below 256 workgroups, quarters
+  // and eighths below 128 (us forward / backward before -> now, bf16: 8
+  // sequences of mean 1,000 x 64 columns 31/18 -> 9/10, 4 x 800 x 512 19/12 ->
+  // 8/10, 8 x 300 x 1,024 13/11 -> 8/8 with half lines against 12/10 at 128;
+  // 12 x 1,000 x 300 fp32 19/28 with half lines, 26/28 with quarters).
+  while (sh.ct > 1 && (int64_t)batch * ((units + sh.ct - 1) / sh.ct) < (sh.ct > 4 ? 256 : 128))
+    sh.ct >>= 1;
   sh.chunks = (units + sh.ct - 1) / sh.ct;
   return sh;
+}
+
+// Dynamic LDS of the kernels, by column lanes and columns per lane.
+inline unsigned sm_fwd_lds(int ct, int vec) {
+  return (unsigned)((2 * (kSmThreadsFwd / 64) * ct + 2 * kSmThreadsFwd) * vec * sizeof(float));
+}
+inline unsigned sm_bwd_lds(int ct, int vec) {
+  return (unsigned)((kSmThreadsBwd / 64) * ct * vec * sizeof(float));
 }
 
 template <typename T>
@@ -457,11 +529,11 @@ int launch_softmax_bwd(const void* y, const void* dy, void* dx, const int32_t* c
     return set_error(SCREE_ERR_INVALID, "scree_varlen_softmax_bwd: grid too large");
   const dim3 grid((unsigned)(batch * sh.chunks));
   if (sh.vec)
-    hipLaunchKernelGGL((varlen_softmax_bwd_kernel<T, V>), grid, dim3(kSmThreadsBwd), 0, stream,
+    hipLaunchKernelGGL((varlen_softmax_bwd_kernel<T, V>), grid, dim3(kSmThreadsBwd), sm_bwd_lds(sh.ct, V), stream,
                        static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<T*>(dx),
                        cu, total, features, sh.ct, (int)sh.chunks);
   else
-    hipLaunchKernelGGL((varlen_softmax_bwd_kernel<T, 1>), grid, dim3(kSmThreadsBwd), 0, stream,
+    hipLaunchKernelGGL((varlen_softmax_bwd_kernel<T, 1>), grid, dim3(kSmThreadsBwd), sm_bwd_lds(sh.ct, 1), stream,
                        static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<T*>(dx),
                        cu, total, features, sh.ct, (int)sh.chunks);
   return check_launch("scree_varlen_softmax_bwd");
@@ -477,11 +549,11 @@ int launch_softmax(const void* x, void* y, const int32_t* cu, int batch, int64_t
     return set_error(SCREE_ERR_INVALID, "scree_varlen_softmax: grid too large");
   const dim3 grid((unsigned)(batch * sh.chunks));
   if (sh.vec)
-    hipLaunchKernelGGL((varlen_softmax_kernel<T, V>), grid, dim3(kSmThreadsFwd), 0, stream,
+    hipLaunchKernelGGL((varlen_softmax_kernel<T, V>), grid, dim3(kSmThreadsFwd), sm_fwd_lds(sh.ct, V), stream,
                        static_cast<const T*>(x), static_cast<T*>(y), cu, total, features, sh.ct,
                        (int)sh.chunks);
   else
-    hipLaunchKernelGGL((varlen_softmax_kernel<T, 1>), grid, dim3(kSmThreadsFwd), 0, stream,
+    hipLaunchKernelGGL((varlen_softmax_kernel<T, 1>), grid, dim3(kSmThreadsFwd), sm_fwd_lds(sh.ct, 1), stream,
                        static_cast<const T*>(x), static_cast<T*>(y), cu, total, features, sh.ct,
                        (int)sh.chunks);
   return check_launch("scree_varlen_softmax");
