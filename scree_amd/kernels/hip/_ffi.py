@@ -8,9 +8,12 @@ entry point raises :class:`HipUnavailableError` -- there is no fallback path.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from pathlib import Path
+
+import torch
 
 _LIB_PATH = Path(os.environ.get("SCREE_HIP_LIB", Path(__file__).resolve().parents[2] / "_lib" / "libscree_hip.so"))
 
@@ -128,16 +131,21 @@ def check(rc: int) -> None:
     raise ScreeHipError(rc, msg)
 
 
-def dtype_code(dtype) -> int:
-    import torch
+_DTYPE_CODES = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
 
-    if dtype == torch.float32:
-        return DTYPE_F32
-    if dtype == torch.float16:
-        return DTYPE_F16
-    if dtype == torch.bfloat16:
-        return DTYPE_BF16
-    raise NotImplementedError(f"dtype {dtype} not supported by the HIP kernels")
+
+def dtype_code(dtype) -> int:
+    code = _DTYPE_CODES.get(dtype)
+    if code is None:
+        raise NotImplementedError(f"dtype {dtype} not supported by the HIP kernels")
+    return code
+
+
+# torch's own accessors for the current device and its raw current stream (what
+# its compiled kernels launch on) cost ~0.3 us against ~2 us for the public paths
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                      lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def stream_of(tensor) -> int:
@@ -145,25 +153,27 @@ def stream_of(tensor) -> int:
     return _raw_stream(tensor.device.index)
 
 
-def _raw_stream_public(index: int) -> int:
-    import torch
-
-    return torch.cuda.current_stream(index).cuda_stream
-
-
-def _pick_raw_stream():
-    # torch's own accessor for the raw current stream (what its compiled
-    # kernels launch on) costs ~0.3 us against ~2 us for the public path
-    import torch
-
-    fn = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    return fn if fn is not None else _raw_stream_public
+def device_guard(device):
+    """``torch.cuda.device(device)``, or a no-op context for a device without an index."""
+    return contextlib.nullcontext() if device.index is None else torch.cuda.device(device)
 
 
-def _raw_stream(index: int) -> int:
-    global _raw_stream
-    _raw_stream = _pick_raw_stream()
-    return _raw_stream(index)
+def launch(fn, tensor, *args) -> None:
+    """``fn(*args, stream)`` with ``tensor``'s device current, on that device's
+    current stream; raises when it reports an error.  Every launch goes
+    through here: no context manager when the device is current already, and
+    one Python call around the library's own (the launchers' share of a small
+    call, more than its GPU time)."""
+    index = tensor.get_device()
+    if index < 0:
+        raise TypeError(f"the HIP kernels need ROCm device tensors, got one on {tensor.device}")
+    if index == _current_device():
+        rc = fn(*args, _raw_stream(index))
+    else:
+        with device_guard(tensor.device):
+            rc = fn(*args, _raw_stream(index))
+    if rc:
+        check(rc)
 
 
 def ptr(tensor) -> int:
@@ -180,15 +190,3 @@ def int64_array(values):
     if cls is None:
         cls = _I64_ARRAYS[n] = ctypes.c_int64 * n
     return cls(*values)
-
-
-def device_guard(device):
-    """``torch.cuda.device(device)`` when another device is current, else a no-op
-    context (entering the real one costs ~5 us per call)."""
-    import contextlib
-
-    import torch
-
-    if device.index is None or torch.cuda.current_device() == device.index:
-        return contextlib.nullcontext()
-    return torch.cuda.device(device)

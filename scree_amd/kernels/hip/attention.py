@@ -35,22 +35,25 @@ import torch
 from . import _ffi
 
 
+_HALF_DTYPES = (torch.float16, torch.bfloat16)
+_ALL_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+
+
 def _check_inputs(q, k, v, allow_fp32: bool = False):
     """The launchers' checks (``triton/varlen_attention.py:213-215``): fp16 or
     bf16, as the reference's GPU launchers; ``allow_fp32`` for the
     Array-level path, which also takes fp32 (computed by the fp32 kernels)."""
-    assert k.shape == v.shape, "k and v must have identical shape"
-    assert q.dim() == 3 and k.dim() == 3, "q, k, v must be (total_tokens, n_heads, head_dim)"
-    assert q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2], (
-        "q, k, v must share total_tokens and head_dim")
-    assert k.shape[1] >= 1 and q.shape[1] % k.shape[1] == 0, (
+    qs, ks = q.shape, k.shape
+    assert ks == v.shape, "k and v must have identical shape"
+    assert len(qs) == 3 and len(ks) == 3, "q, k, v must be (total_tokens, n_heads, head_dim)"
+    assert qs[0] == ks[0] and qs[2] == ks[2], "q, k, v must share total_tokens and head_dim"
+    assert ks[1] >= 1 and qs[1] % ks[1] == 0, (
         "k/v heads must divide q heads (grouped-query attention)")
     assert q.is_cuda, "varlen_attention_hip requires ROCm device tensors"
-    dtypes = (torch.float16, torch.bfloat16, torch.float32) if allow_fp32 else (torch.float16,
-                                                                               torch.bfloat16)
-    assert q.dtype in dtypes, "fp16 or bf16 only" if not allow_fp32 else "fp16, bf16 or fp32 only"
-    assert q.dtype == k.dtype == v.dtype, "q, k, v must share a dtype"
-    assert q.dim() == 3, "q, k, v must be (total_tokens, n_heads, head_dim)"
+    dtype = q.dtype
+    assert dtype in _ALL_DTYPES if allow_fp32 else dtype in _HALF_DTYPES, (
+        "fp16, bf16 or fp32 only" if allow_fp32 else "fp16 or bf16 only")
+    assert dtype == k.dtype == v.dtype, "q, k, v must share a dtype"
 
 
 # Row and head strides the kernels index with 32-bit element offsets.
@@ -144,10 +147,8 @@ def attention_schedule(cu_seqlens: torch.Tensor, total_tokens: int, head_dim: in
     nbytes = workspace_bytes(batch, total_tokens, head_dim)
     if workspace is None:
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=cu_seqlens.device)
-    with _ffi.device_guard(cu_seqlens.device):
-        _ffi.check(lib.scree_attn_schedule(
-            _ffi.ptr(cu_seqlens), batch, total_tokens, head_dim, int(bool(causal)),
-            _ffi.ptr(workspace), workspace.numel(), _ffi.stream_of(cu_seqlens)))
+    _ffi.launch(lib.scree_attn_schedule, cu_seqlens, cu_seqlens.data_ptr(), batch, total_tokens,
+                head_dim, int(bool(causal)), workspace.data_ptr(), workspace.numel())
     return workspace
 
 
@@ -171,11 +172,10 @@ def _attn_fwd(q, k, v, cu, causal, out, lse, workspace):
     lib = _ffi.lib()
     total, heads, head_dim = q.shape
     strides = _ffi.int64_array(q.stride()[:2] + k.stride()[:2] + v.stride()[:2] + out.stride()[:2])
-    _ffi.check(lib.scree_attn_fwd_gqa(
-        _ffi.ptr(q), _ffi.ptr(k), _ffi.ptr(v), _ffi.ptr(out), _ffi.ptr(lse), _ffi.ptr(cu),
-        cu.numel() - 1, total, heads, k.shape[1], head_dim, strides, 1.0 / math.sqrt(head_dim),
-        int(bool(causal)), _ffi.dtype_code(q.dtype), _ffi.ptr(workspace), workspace.numel(),
-        _ffi.stream_of(q)))
+    _ffi.launch(lib.scree_attn_fwd_gqa, q, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                out.data_ptr(), lse.data_ptr(), cu.data_ptr(), cu.numel() - 1, total, heads,
+                k.shape[1], head_dim, strides, 1.0 / math.sqrt(head_dim), int(bool(causal)),
+                _ffi.dtype_code(q.dtype), workspace.data_ptr(), workspace.numel())
 
 
 def _attn_bwd(do, q, k, v, o, lse, cu, causal, dq, dk, dv, delta, workspace):
@@ -183,34 +183,33 @@ def _attn_bwd(do, q, k, v, o, lse, cu, causal, dq, dk, dv, delta, workspace):
     total, heads, head_dim = q.shape
     ts = (do, q, k, v, o, dq, dk, dv)
     strides = _ffi.int64_array(sum((t.stride()[:2] for t in ts), ()))
-    _ffi.check(lib.scree_attn_bwd_gqa(
-        _ffi.ptr(do), _ffi.ptr(q), _ffi.ptr(k), _ffi.ptr(v), _ffi.ptr(o), _ffi.ptr(lse),
-        _ffi.ptr(dq), _ffi.ptr(dk), _ffi.ptr(dv), _ffi.ptr(delta), _ffi.ptr(cu),
-        cu.numel() - 1, total, heads, k.shape[1], head_dim, strides, 1.0 / math.sqrt(head_dim),
-        int(bool(causal)), _ffi.dtype_code(q.dtype), _ffi.ptr(workspace), workspace.numel(),
-        _ffi.stream_of(q)))
+    _ffi.launch(lib.scree_attn_bwd_gqa, q, *[t.data_ptr() for t in (do, q, k, v, o, lse, dq, dk,
+                                                                    dv, delta, cu)],
+                cu.numel() - 1, total, heads, k.shape[1], head_dim, strides,
+                1.0 / math.sqrt(head_dim), int(bool(causal)), _ffi.dtype_code(q.dtype),
+                workspace.data_ptr(), workspace.numel())
 
 
 def _attn_bwd_dq(do, q, k, v, o, lse, cu, causal, dq, delta, workspace):
     lib = _ffi.lib()
     total, heads, head_dim = q.shape
     strides = _ffi.int64_array(sum((t.stride()[:2] for t in (do, q, k, v, o, dq)), ()))
-    _ffi.check(lib.scree_attn_bwd_dq_gqa(
-        _ffi.ptr(do), _ffi.ptr(q), _ffi.ptr(k), _ffi.ptr(v), _ffi.ptr(o), _ffi.ptr(lse),
-        _ffi.ptr(dq), _ffi.ptr(delta), _ffi.ptr(cu), cu.numel() - 1, total, heads, k.shape[1],
-        head_dim, strides, 1.0 / math.sqrt(head_dim), int(bool(causal)),
-        _ffi.dtype_code(q.dtype), _ffi.ptr(workspace), workspace.numel(), _ffi.stream_of(q)))
+    _ffi.launch(lib.scree_attn_bwd_dq_gqa, q,
+                *[t.data_ptr() for t in (do, q, k, v, o, lse, dq, delta, cu)],
+                cu.numel() - 1, total, heads, k.shape[1], head_dim, strides,
+                1.0 / math.sqrt(head_dim), int(bool(causal)), _ffi.dtype_code(q.dtype),
+                workspace.data_ptr(), workspace.numel())
 
 
 def _attn_bwd_dkv(do, q, k, v, lse, delta, cu, causal, dk, dv, workspace):
     lib = _ffi.lib()
     total, heads, head_dim = q.shape
     strides = _ffi.int64_array(sum((t.stride()[:2] for t in (do, q, k, v, dk, dv)), ()))
-    _ffi.check(lib.scree_attn_bwd_dkv_gqa(
-        _ffi.ptr(do), _ffi.ptr(q), _ffi.ptr(k), _ffi.ptr(v), _ffi.ptr(lse), _ffi.ptr(delta),
-        _ffi.ptr(dk), _ffi.ptr(dv), _ffi.ptr(cu), cu.numel() - 1, total, heads, k.shape[1],
-        head_dim, strides, 1.0 / math.sqrt(head_dim), int(bool(causal)),
-        _ffi.dtype_code(q.dtype), _ffi.ptr(workspace), workspace.numel(), _ffi.stream_of(q)))
+    _ffi.launch(lib.scree_attn_bwd_dkv_gqa, q,
+                *[t.data_ptr() for t in (do, q, k, v, lse, delta, dk, dv, cu)],
+                cu.numel() - 1, total, heads, k.shape[1], head_dim, strides,
+                1.0 / math.sqrt(head_dim), int(bool(causal)), _ffi.dtype_code(q.dtype),
+                workspace.data_ptr(), workspace.numel())
 
 
 def varlen_attention_hip(q, k, v, cu_seqlens, causal: bool = False, block_m: int = 64,
@@ -245,10 +244,9 @@ def varlen_attention_hip(q, k, v, cu_seqlens, causal: bool = False, block_m: int
     cu = _cu(cu_seqlens, q.device)
     qk, kk, vk = _kernel_view(q), _kernel_view(k), _kernel_view(v)
     ok = _kernel_view(out)
-    with _ffi.device_guard(q.device):
-        if workspace is None:
-            workspace = prepare_workspace(cu, total, head_dim, causal, n_heads)
-        _attn_fwd(qk, kk, vk, cu, causal, ok, lse, workspace)
+    if workspace is None:
+        workspace = prepare_workspace(cu, total, head_dim, causal, n_heads)
+    _attn_fwd(qk, kk, vk, cu, causal, ok, lse, workspace)
     if ok is not out:
         out.copy_(ok)
     if return_lse:
@@ -284,10 +282,9 @@ def varlen_attention_hip_backward(do, q, k, v, o, lse, cu_seqlens, causal: bool 
         assert delta_buffer.is_contiguous(), "delta_buffer must be contiguous"
         delta = delta_buffer
     ins = [_kernel_view(t) for t in (do, q, k, v, o)]
-    with _ffi.device_guard(q.device):
-        if workspace is None:
-            workspace = prepare_workspace(cu, total, head_dim, causal, n_heads,
-                                          _bwd_workspace(cu, total, n_heads, k.shape[1], head_dim),
-                                          for_backward=True)
-        _attn_bwd(*ins, lse.contiguous(), cu, causal, dq, dk, dv, delta, workspace)
+    if workspace is None:
+        workspace = prepare_workspace(cu, total, head_dim, causal, n_heads,
+                                      _bwd_workspace(cu, total, n_heads, k.shape[1], head_dim),
+                                      for_backward=True)
+    _attn_bwd(*ins, lse.contiguous(), cu, causal, dq, dk, dv, delta, workspace)
     return dq, dk, dv

@@ -21,15 +21,25 @@ launchers are :func:`varlen_rmsnorm_hip_backward` and
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _ffi
+
+_CODE_DTYPES = {code: dtype for dtype, code in _ffi._DTYPE_CODES.items()}
 
 
 def _flat(x):
     assert x.is_cuda, "varlen norms on HIP require ROCm device tensors"
     d = x.shape[-1]
+    if x.dim() == 2 and x.is_contiguous():
+        return x, d
     return x.reshape(-1, d).contiguous(), d
+
+
+def _like(y2, shape):
+    return y2 if y2.shape == shape else y2.reshape(shape)
 
 
 def _param(p, d, device, dtype, name):
@@ -41,17 +51,15 @@ def _param(p, d, device, dtype, name):
 
 
 def _dparam_code(p):
-    return _ffi.dtype_code(p.dtype) if p.dtype in (torch.float32, torch.float16, torch.bfloat16) else _ffi.DTYPE_F32
+    return _ffi._DTYPE_CODES.get(p.dtype, _ffi.DTYPE_F32)
 
 
 def rmsnorm_fwd(x2, w, eps, want_stats):
     rows, d = x2.shape
     y = torch.empty_like(x2)
     rstd = torch.empty(rows, dtype=torch.float32, device=x2.device) if want_stats else None
-    with _ffi.device_guard(x2.device):
-        _ffi.check(_ffi.lib().scree_rmsnorm_fwd(
-            _ffi.ptr(x2), _ffi.ptr(w), _ffi.ptr(y), _ffi.ptr(rstd), rows, d, float(eps),
-            _ffi.dtype_code(x2.dtype), _ffi.stream_of(x2)))
+    _ffi.launch(_ffi.lib().scree_rmsnorm_fwd, x2, x2.data_ptr(), _ffi.ptr(w), y.data_ptr(),
+                _ffi.ptr(rstd), rows, d, float(eps), _ffi.dtype_code(x2.dtype))
     return y, rstd
 
 
@@ -61,33 +69,35 @@ def layernorm_fwd(x2, w, b, eps, want_stats):
     mean = rstd = None
     if want_stats:
         mean = torch.empty(rows, dtype=torch.float32, device=x2.device)
-        rstd = torch.empty(rows, dtype=torch.float32, device=x2.device)
-    with _ffi.device_guard(x2.device):
-        _ffi.check(_ffi.lib().scree_layernorm_fwd(
-            _ffi.ptr(x2), _ffi.ptr(w), _ffi.ptr(b), _ffi.ptr(y), _ffi.ptr(mean), _ffi.ptr(rstd),
-            rows, d, float(eps), _ffi.dtype_code(x2.dtype), _ffi.stream_of(x2)))
+        rstd = torch.empty_like(mean)
+    _ffi.launch(_ffi.lib().scree_layernorm_fwd, x2, x2.data_ptr(), _ffi.ptr(w), _ffi.ptr(b),
+                y.data_ptr(), _ffi.ptr(mean), _ffi.ptr(rstd), rows, d, float(eps),
+                _ffi.dtype_code(x2.dtype))
     return y, mean, rstd
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(rows, d):
+    return max(int(_ffi.lib().scree_norm_bwd_workspace_bytes(rows, d)), 16)
+
+
 def _workspace(rows, d, device):
-    n = int(_ffi.lib().scree_norm_bwd_workspace_bytes(rows, d))
-    return torch.empty(max(n, 16), dtype=torch.uint8, device=device)
+    """Room for the partial parameter gradients (only a call that wants them needs it)."""
+    return torch.empty(_workspace_bytes(rows, d), dtype=torch.uint8, device=device)
 
 
 def rmsnorm_bwd(dy2, x2, w, rstd, want_dw, dw_like=None):
     rows, d = x2.shape
     dx = torch.empty_like(x2)
-    dw = None
-    code = _ffi.DTYPE_F32
+    dw, code, ws, nws = None, _ffi.DTYPE_F32, None, 0
     if want_dw:
         code = _dparam_code(dw_like) if dw_like is not None else _ffi.DTYPE_F32
-        dw = torch.empty(d, dtype=_code_dtype(code), device=x2.device)
-    ws = _workspace(rows, d, x2.device)
-    with _ffi.device_guard(x2.device):
-        _ffi.check(_ffi.lib().scree_rmsnorm_bwd(
-            _ffi.ptr(dy2), _ffi.ptr(x2), _ffi.ptr(w), _ffi.ptr(rstd), _ffi.ptr(dx), _ffi.ptr(dw),
-            code, rows, d, _ffi.dtype_code(x2.dtype), _ffi.ptr(ws), ws.numel(),
-            _ffi.stream_of(x2)))
+        dw = torch.empty(d, dtype=_CODE_DTYPES[code], device=x2.device)
+        ws = _workspace(rows, d, x2.device)
+        nws = ws.numel()
+    _ffi.launch(_ffi.lib().scree_rmsnorm_bwd, x2, dy2.data_ptr(), x2.data_ptr(), _ffi.ptr(w),
+                rstd.data_ptr(), dx.data_ptr(), _ffi.ptr(dw), code, rows, d,
+                _ffi.dtype_code(x2.dtype), _ffi.ptr(ws), nws)
     return dx, dw
 
 
@@ -95,14 +105,18 @@ def layernorm_bwd(dy2, x2, w, mean, rstd, want_dw, want_db, p_like=None):
     rows, d = x2.shape
     dx = torch.empty_like(x2)
     code = _dparam_code(p_like) if p_like is not None else _ffi.DTYPE_F32
-    dw = torch.empty(d, dtype=_code_dtype(code), device=x2.device) if want_dw else None
-    db = torch.empty(d, dtype=_code_dtype(code), device=x2.device) if want_db else None
-    ws = _workspace(rows, d, x2.device)
-    with _ffi.device_guard(x2.device):
-        _ffi.check(_ffi.lib().scree_layernorm_bwd(
-            _ffi.ptr(dy2), _ffi.ptr(x2), _ffi.ptr(w), _ffi.ptr(mean), _ffi.ptr(rstd),
-            _ffi.ptr(dx), _ffi.ptr(dw), _ffi.ptr(db), code, rows, d, _ffi.dtype_code(x2.dtype),
-            _ffi.ptr(ws), ws.numel(), _ffi.stream_of(x2)))
+    dw = db = ws = None
+    nws = 0
+    if want_dw:
+        dw = torch.empty(d, dtype=_CODE_DTYPES[code], device=x2.device)
+    if want_db:
+        db = torch.empty(d, dtype=_CODE_DTYPES[code], device=x2.device)
+    if want_dw or want_db:
+        ws = _workspace(rows, d, x2.device)
+        nws = ws.numel()
+    _ffi.launch(_ffi.lib().scree_layernorm_bwd, x2, dy2.data_ptr(), x2.data_ptr(), _ffi.ptr(w),
+                mean.data_ptr(), rstd.data_ptr(), dx.data_ptr(), _ffi.ptr(dw), _ffi.ptr(db), code,
+                rows, d, _ffi.dtype_code(x2.dtype), _ffi.ptr(ws), nws)
     return dx, dw, db
 
 
@@ -111,33 +125,25 @@ def add_rmsnorm_fwd(x2, r2, w, eps, want_stats):
     h = torch.empty_like(x2)
     y = torch.empty_like(x2)
     rstd = torch.empty(rows, dtype=torch.float32, device=x2.device) if want_stats else None
-    with _ffi.device_guard(x2.device):
-        _ffi.check(_ffi.lib().scree_add_rmsnorm_fwd(
-            _ffi.ptr(x2), _ffi.ptr(r2), _ffi.ptr(w), _ffi.ptr(h), _ffi.ptr(y), _ffi.ptr(rstd),
-            rows, d, float(eps), _ffi.dtype_code(x2.dtype), _ffi.stream_of(x2)))
+    _ffi.launch(_ffi.lib().scree_add_rmsnorm_fwd, x2, x2.data_ptr(), r2.data_ptr(), _ffi.ptr(w),
+                h.data_ptr(), y.data_ptr(), _ffi.ptr(rstd), rows, d, float(eps),
+                _ffi.dtype_code(x2.dtype))
     return h, y, rstd
 
 
 def add_rmsnorm_bwd(dy2, dh2, h2, w, rstd, want_dw, dw_like=None):
     rows, d = h2.shape
     dx = torch.empty_like(h2)
-    dw = None
-    code = _ffi.DTYPE_F32
+    dw, code, ws, nws = None, _ffi.DTYPE_F32, None, 0
     if want_dw:
         code = _dparam_code(dw_like) if dw_like is not None else _ffi.DTYPE_F32
-        dw = torch.empty(d, dtype=_code_dtype(code), device=h2.device)
-    ws = _workspace(rows, d, h2.device)
-    with _ffi.device_guard(h2.device):
-        _ffi.check(_ffi.lib().scree_add_rmsnorm_bwd(
-            _ffi.ptr(dy2), _ffi.ptr(dh2), _ffi.ptr(h2), _ffi.ptr(w), _ffi.ptr(rstd), _ffi.ptr(dx),
-            _ffi.ptr(dw), code, rows, d, _ffi.dtype_code(h2.dtype), _ffi.ptr(ws), ws.numel(),
-            _ffi.stream_of(h2)))
+        dw = torch.empty(d, dtype=_CODE_DTYPES[code], device=h2.device)
+        ws = _workspace(rows, d, h2.device)
+        nws = ws.numel()
+    _ffi.launch(_ffi.lib().scree_add_rmsnorm_bwd, h2, dy2.data_ptr(), _ffi.ptr(dh2), h2.data_ptr(),
+                _ffi.ptr(w), rstd.data_ptr(), dx.data_ptr(), _ffi.ptr(dw), code, rows, d,
+                _ffi.dtype_code(h2.dtype), _ffi.ptr(ws), nws)
     return dx, dw
-
-
-def _code_dtype(code):
-    return {_ffi.DTYPE_F32: torch.float32, _ffi.DTYPE_F16: torch.float16,
-            _ffi.DTYPE_BF16: torch.bfloat16}[code]
 
 
 class _RMSNormFn(torch.autograd.Function):
@@ -148,17 +154,17 @@ class _RMSNormFn(torch.autograd.Function):
         y, rstd = rmsnorm_fwd(x2, w, eps, want_stats=True)
         ctx.save_for_backward(x2, w, rstd, weight)
         ctx.shape = x.shape
-        return y.reshape(x.shape)
+        return _like(y, x.shape)
 
     @staticmethod
     def backward(ctx, dy):
         x2, w, rstd, weight = ctx.saved_tensors
-        dy2 = dy.reshape(x2.shape).contiguous()
+        dy2 = _like(dy, x2.shape).contiguous()
         want_dw = weight is not None and ctx.needs_input_grad[1]
         dx, dw = rmsnorm_bwd(dy2, x2, w, rstd, want_dw, dw_like=weight)
         if dw is not None and dw.dtype != weight.dtype:
             dw = dw.to(weight.dtype)
-        return dx.reshape(ctx.shape), dw, None
+        return _like(dx, ctx.shape), dw, None
 
 
 class _LayerNormFn(torch.autograd.Function):
@@ -170,12 +176,12 @@ class _LayerNormFn(torch.autograd.Function):
         y, mean, rstd = layernorm_fwd(x2, w, b, eps, want_stats=True)
         ctx.save_for_backward(x2, w, mean, rstd, weight, bias)
         ctx.shape = x.shape
-        return y.reshape(x.shape)
+        return _like(y, x.shape)
 
     @staticmethod
     def backward(ctx, dy):
         x2, w, mean, rstd, weight, bias = ctx.saved_tensors
-        dy2 = dy.reshape(x2.shape).contiguous()
+        dy2 = _like(dy, x2.shape).contiguous()
         want_dw = weight is not None and ctx.needs_input_grad[1]
         want_db = bias is not None and ctx.needs_input_grad[2]
         like = weight if weight is not None else bias
@@ -184,7 +190,7 @@ class _LayerNormFn(torch.autograd.Function):
             dw = dw.to(weight.dtype)
         if db is not None and db.dtype != bias.dtype:
             db = db.to(bias.dtype)
-        return dx.reshape(ctx.shape), dw, db, None
+        return _like(dx, ctx.shape), dw, db, None
 
 
 class _AddRMSNormFn(torch.autograd.Function):
@@ -196,18 +202,18 @@ class _AddRMSNormFn(torch.autograd.Function):
         h, y, rstd = add_rmsnorm_fwd(x2, r2, w, eps, want_stats=True)
         ctx.save_for_backward(h, w, rstd, weight)
         ctx.shape = x.shape
-        return h.reshape(x.shape), y.reshape(x.shape)
+        return _like(h, x.shape), _like(y, x.shape)
 
     @staticmethod
     def backward(ctx, dh, dy):
         h2, w, rstd, weight = ctx.saved_tensors
         want_dw = weight is not None and ctx.needs_input_grad[2]
-        dy2 = (torch.zeros_like(h2) if dy is None else dy.reshape(h2.shape).contiguous())
-        dh2 = None if dh is None else dh.reshape(h2.shape).contiguous()
+        dy2 = (torch.zeros_like(h2) if dy is None else _like(dy, h2.shape).contiguous())
+        dh2 = None if dh is None else _like(dh, h2.shape).contiguous()
         dx, dw = add_rmsnorm_bwd(dy2, dh2, h2, w, rstd, want_dw, dw_like=weight)
         if dw is not None and dw.dtype != weight.dtype:
             dw = dw.to(weight.dtype)
-        dx = dx.reshape(ctx.shape)
+        dx = _like(dx, ctx.shape)
         # x and residual receive the same gradient (as torch's own add backward does)
         return dx, dx, dw, None
 
@@ -223,7 +229,7 @@ def varlen_rmsnorm_hip(x, weight=None, eps: float = 1e-6):
     x2, d = _flat(x)
     w = _param(weight, d, x.device, x.dtype, "weight")
     y, _ = rmsnorm_fwd(x2, w, eps, want_stats=False)
-    return y.reshape(x.shape)
+    return _like(y, x.shape)
 
 
 def varlen_layernorm_hip(x, weight=None, bias=None, eps: float = 1e-5):
@@ -234,7 +240,7 @@ def varlen_layernorm_hip(x, weight=None, bias=None, eps: float = 1e-5):
     w = _param(weight, d, x.device, x.dtype, "weight")
     b = _param(bias, d, x.device, x.dtype, "bias")
     y, _, _ = layernorm_fwd(x2, w, b, eps, want_stats=False)
-    return y.reshape(x.shape)
+    return _like(y, x.shape)
 
 
 def varlen_add_rmsnorm_hip(x, residual, weight=None, eps: float = 1e-6):
@@ -255,7 +261,7 @@ def varlen_add_rmsnorm_hip(x, residual, weight=None, eps: float = 1e-6):
     r2, _ = _flat(residual)
     w = _param(weight, d, x.device, x.dtype, "weight")
     h, y, _ = add_rmsnorm_fwd(x2, r2, w, eps, want_stats=False)
-    return h.reshape(x.shape), y.reshape(x.shape)
+    return _like(h, x.shape), _like(y, x.shape)
 
 
 def varlen_add_rmsnorm_hip_backward(dy, dh, h, weight=None, eps: float = 1e-6, rstd=None):
@@ -265,10 +271,10 @@ def varlen_add_rmsnorm_hip_backward(dy, dh, h, weight=None, eps: float = 1e-6, r
     w = _param(weight, d, h.device, h.dtype, "weight")
     if rstd is None:
         _, rstd = rmsnorm_fwd(h2, w, eps, want_stats=True)
-    dh2 = None if dh is None else dh.reshape(h2.shape).contiguous()
-    dx, dw = add_rmsnorm_bwd(dy.reshape(h2.shape).contiguous(), dh2, h2, w,
+    dh2 = None if dh is None else _like(dh, h2.shape).contiguous()
+    dx, dw = add_rmsnorm_bwd(_like(dy, h2.shape).contiguous(), dh2, h2, w,
                              rstd.reshape(-1).contiguous(), weight is not None, dw_like=weight)
-    return dx.reshape(h.shape), dw
+    return _like(dx, h.shape), dw
 
 
 def varlen_rmsnorm_hip_autograd(x, weight=None, eps: float = 1e-6):
@@ -286,9 +292,9 @@ def varlen_rmsnorm_hip_backward(dy, x, weight=None, eps: float = 1e-6, rstd=None
     w = _param(weight, d, x.device, x.dtype, "weight")
     if rstd is None:
         _, rstd = rmsnorm_fwd(x2, w, eps, want_stats=True)
-    dx, dw = rmsnorm_bwd(dy.reshape(x2.shape).contiguous(), x2, w, rstd.reshape(-1).contiguous(),
+    dx, dw = rmsnorm_bwd(_like(dy, x2.shape).contiguous(), x2, w, rstd.reshape(-1).contiguous(),
                          weight is not None, dw_like=weight)
-    return dx.reshape(x.shape), dw
+    return _like(dx, x.shape), dw
 
 
 def varlen_layernorm_hip_backward(dy, x, weight=None, bias=None, eps: float = 1e-5, mean=None,
@@ -299,7 +305,7 @@ def varlen_layernorm_hip_backward(dy, x, weight=None, bias=None, eps: float = 1e
     if mean is None or rstd is None:
         _, mean, rstd = layernorm_fwd(x2, w, None, eps, want_stats=True)
     like = weight if weight is not None else bias
-    dx, dw, db = layernorm_bwd(dy.reshape(x2.shape).contiguous(), x2, w,
+    dx, dw, db = layernorm_bwd(_like(dy, x2.shape).contiguous(), x2, w,
                                mean.reshape(-1).contiguous(), rstd.reshape(-1).contiguous(),
                                weight is not None, bias is not None, p_like=like)
-    return dx.reshape(x.shape), dw, db
+    return _like(dx, x.shape), dw, db

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 
+import numpy as np
 import torch
 
 from . import _ffi
@@ -48,18 +49,15 @@ def to_padded_hip(values, offsets, side="right", fill_value=0.0, max_len=None):
     batch = off.numel() - 1
     assert batch >= 1, "offsets must have batch + 1 entries"
     if max_len is None:
-        host = off.cpu()
-        max_len = int((host[1:] - host[:-1]).max()) if batch > 0 else 0
+        max_len = int(np.diff(off.cpu().numpy()).max())
     feat = tuple(values.shape[1:])
     vals = values.contiguous()
     padded = torch.empty((batch, max_len, *feat), dtype=vals.dtype, device=vals.device)
     mask = torch.empty((batch, max_len), dtype=torch.bool, device=vals.device)
     fill, elem = _fill_bytes(fill_value, vals.dtype)
-    with _ffi.device_guard(vals.device):
-        _ffi.check(_ffi.lib().scree_to_padded(
-            _ffi.ptr(vals), _ffi.ptr(off), batch, vals.shape[0], max_len, _row_bytes(vals, 1),
-            1 if side == "left" else 0, ctypes.cast(fill, ctypes.c_void_p), elem,
-            _ffi.ptr(padded), _ffi.ptr(mask), _ffi.stream_of(vals)))
+    _ffi.launch(_ffi.lib().scree_to_padded, vals, vals.data_ptr(), off.data_ptr(), batch,
+                vals.shape[0], max_len, _row_bytes(vals, 1), 1 if side == "left" else 0,
+                ctypes.cast(fill, ctypes.c_void_p), elem, padded.data_ptr(), mask.data_ptr())
     return padded, mask
 
 
@@ -82,16 +80,13 @@ def from_padded_hip(padded, mask, total=None):
     m = mask.to(device=padded.device, dtype=torch.bool).contiguous()
     pad = padded.contiguous()
     offsets = torch.empty(batch + 1, dtype=torch.int32, device=pad.device)
-    with _ffi.device_guard(pad.device):
-        _ffi.check(_ffi.lib().scree_padded_offsets(
-            _ffi.ptr(m), batch, t, _ffi.ptr(offsets), _ffi.stream_of(pad)))
-        if total is None:
-            total = int(offsets[-1].item())
-        total = int(total)
-        if total < 0:
-            raise ValueError(f"total must be non-negative, got {total}")
-        values = torch.empty((total, *pad.shape[2:]), dtype=pad.dtype, device=pad.device)
-        _ffi.check(_ffi.lib().scree_from_padded(
-            _ffi.ptr(pad), _ffi.ptr(offsets), batch, t, _row_bytes(pad, 2), total,
-            _ffi.ptr(values), _ffi.stream_of(pad)))
+    _ffi.launch(_ffi.lib().scree_padded_offsets, pad, m.data_ptr(), batch, t, offsets.data_ptr())
+    if total is None:
+        total = int(offsets[-1].item())
+    total = int(total)
+    if total < 0:
+        raise ValueError(f"total must be non-negative, got {total}")
+    values = torch.empty((total, *pad.shape[2:]), dtype=pad.dtype, device=pad.device)
+    _ffi.launch(_ffi.lib().scree_from_padded, pad, pad.data_ptr(), offsets.data_ptr(), batch, t,
+                _row_bytes(pad, 2), total, values.data_ptr())
     return values, offsets

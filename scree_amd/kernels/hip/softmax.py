@@ -41,10 +41,9 @@ def softmax_fwd(x, cu_seqlens, out=None):
     f = _features(xc)
     if xc.numel() == 0:
         return y
-    with _ffi.device_guard(xc.device):
-        _ffi.check(_ffi.lib().scree_varlen_softmax(
-            _ffi.ptr(xc), _ffi.ptr(y), _ffi.ptr(cu_seqlens), cu_seqlens.numel() - 1,
-            xc.shape[0], f, _ffi.dtype_code(xc.dtype), _ffi.stream_of(xc)))
+    _ffi.launch(_ffi.lib().scree_varlen_softmax, xc, xc.data_ptr(), y.data_ptr(),
+                cu_seqlens.data_ptr(), cu_seqlens.numel() - 1, xc.shape[0], f,
+                _ffi.dtype_code(xc.dtype))
     return y
 
 
@@ -53,10 +52,9 @@ def softmax_bwd(y, dy, cu_seqlens):
     dx = torch.empty_like(yc)
     if yc.numel() == 0:
         return dx
-    with _ffi.device_guard(yc.device):
-        _ffi.check(_ffi.lib().scree_varlen_softmax_bwd(
-            _ffi.ptr(yc), _ffi.ptr(dyc), _ffi.ptr(dx), _ffi.ptr(cu_seqlens), cu_seqlens.numel() - 1,
-            yc.shape[0], _features(yc), _ffi.dtype_code(yc.dtype), _ffi.stream_of(yc)))
+    _ffi.launch(_ffi.lib().scree_varlen_softmax_bwd, yc, yc.data_ptr(), dyc.data_ptr(),
+                dx.data_ptr(), cu_seqlens.data_ptr(), cu_seqlens.numel() - 1, yc.shape[0],
+                _features(yc), _ffi.dtype_code(yc.dtype))
     return dx
 
 
