@@ -8,9 +8,10 @@
 // of the row in registers (dim = CHUNKS * 64 lanes * 16 bytes at most), so x
 // is read from HBM exactly once; the reductions are wave-wide shuffles.  Rows
 // of at most 128 vectors take 4 to 64 lanes each (short rows, below).
-// Generic path (dim not a multiple of one 16-byte vector, unaligned buffers,
-// or rows longer than the fast path holds): one wavefront per row looping
-// over the columns.
+// Rows that are not whole vectors, and unaligned buffers, run the same kernels
+// with element-aligned vectors (odd widths, below).  Generic path (rows shorter
+// than one vector or longer than the fast path holds): one wavefront per row
+// looping over the columns.
 //
 // Backward (norm_bwd_cols): each thread of a block (or, at up to 256 vectors
 // per row, of a team of waves in it) owns fixed 16-byte column vectors across
@@ -33,6 +34,62 @@ constexpr int kFwdWaves = 4;       // rows (waves) per forward block
 constexpr int kMaxParts = 512;     // partial rows of a backward, at most
 constexpr int kMaxChunks = 16;     // 16-byte vectors per lane on the fast path
 
+// --------------------------------------------------------------- odd widths
+// ODD kernels take rows that are not whole 16-byte vectors, or buffers that are
+// not 16-byte aligned: vectors are read and written at element alignment (the
+// hardware takes any, and a row's unaligned vectors still cover whole cache
+// lines between them), and the last vector of a row is moved back to end with
+// it.  Its first `dup` elements are then also the previous vector's: both lanes
+// compute and store the same values, and only the sums leave them out.
+// Scalar loops over the columns, which these replace, were bound by the issue
+// of 2-byte loads.  RMSNorm / LayerNorm / add+RMSNorm, us, before -> now:
+// 12,160 x 1,001 bf16 forward 27/39/36 -> 11/13/20, backward 90/91/100 ->
+// 22/26/26; 12,160 x 4,095 bf16 forward 137/195/184 -> 37/45/70, backward
+// 269/271/351 -> 61/71/83; 1,000 x 130 fp16 backward 15/16/15 -> 7/8/7.
+typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+template <typename T, bool ODD>
+struct RowVec {
+  static constexpr int VEC = 16 / sizeof(T);
+  typedef typename std::conditional<sizeof(T) == 2, u32x4_a2, u32x4_a4>::type u32x4e;
+  int nvec, dim;
+  __device__ __forceinline__ explicit RowVec(int d) : nvec(ODD ? (d + VEC - 1) / VEC : d / VEC), dim(d) {}
+  // column of vector v's first element, and how many of its elements repeat
+  __device__ __forceinline__ int col(int v) const { return ODD ? min(v * VEC, dim - VEC) : v * VEC; }
+  __device__ __forceinline__ int dup(int v) const { return ODD && v == nvec - 1 ? nvec * VEC - dim : 0; }
+  static __device__ __forceinline__ bool counts(int e, int dup) { return !ODD || e >= dup; }
+  static __device__ __forceinline__ uint4 ld(const T* p) {
+    if constexpr (!ODD) return ld16(p);
+    const u32x4e v = *reinterpret_cast<const u32x4e*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+  }
+  static __device__ __forceinline__ uint4 ld_nt(const T* p) {
+    if constexpr (!ODD) return ld16_nt(p);
+    const u32x4e v = __builtin_nontemporal_load(reinterpret_cast<const u32x4e*>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+  }
+  static __device__ __forceinline__ void st_nt(T* p, const uint4& v) {
+    if constexpr (!ODD) {
+      st16_nt(p, v);
+    } else {
+      const u32x4e u = {v.x, v.y, v.z, v.w};
+      __builtin_nontemporal_store(u, reinterpret_cast<u32x4e*>(p));
+    }
+  }
+  // For rows past 128 vectors: a wide odd row's vectors straddle cache lines
+  // that the next instruction completes, which plain stores leave in L2 until
+  // then (add+RMSNorm, 12,160 x 4,095 bf16: 70 us against 85 nontemporal; on
+  // rows of 770 nontemporal is the faster, 10.3 against 12.0 for LayerNorm).
+  static __device__ __forceinline__ void st_wide(T* p, const uint4& v) {
+    if constexpr (!ODD) {
+      st16_nt(p, v);
+    } else {
+      const u32x4e u = {v.x, v.y, v.z, v.w};
+      *reinterpret_cast<u32x4e*>(p) = u;
+    }
+  }
+};
+
 // ------------------------------------------------------------------ forward
 // RES (RMSNorm only): the normalised row is h = x + res, rounded to T as a
 // separate addition would round it; h is written out and normalised.
@@ -45,7 +102,7 @@ constexpr int kLnWaves = 8;
 template <bool LAYER>
 constexpr int fwd_waves() { return LAYER ? kLnWaves : kFwdWaves; }
 
-template <typename T, int CHUNKS, bool LAYER, bool RES>
+template <typename T, int CHUNKS, bool LAYER, bool RES, bool ODD>
 __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_vec(
     const T* __restrict__ x, const T* __restrict__ res, const T* __restrict__ w,
     const T* __restrict__ b, T* __restrict__ hout, T* __restrict__ y,
@@ -55,13 +112,15 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t row = (int64_t)blockIdx.x * WAVES + (threadIdx.x / kWave);
   const bool live = row < rows;
-  const int nvec = dim / VEC;
+  typedef RowVec<T, ODD> RV;
+  const RV rv(dim);
+  const int nvec = rv.nvec;
   const T* xr = x + row * (int64_t)dim;
   uint4 v[CHUNKS];
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int vi = c * kWave + lane;
-    v[c] = live && vi < nvec ? ld16_nt(xr + (int64_t)vi * VEC) : make_uint4(0, 0, 0, 0);
+    v[c] = live && vi < nvec ? RV::ld_nt(xr + rv.col(vi)) : make_uint4(0, 0, 0, 0);
   }
   // LayerNorm: the block copies the weight and bias rows into LDS while its
   // rows load (one L2 read per block instead of per row, and off the
@@ -70,8 +129,8 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
   __shared__ __align__(16) T wb[2 * NMAX];
   if constexpr (LAYER) {
     for (int vi = threadIdx.x; vi < nvec; vi += WAVES * kWave) {
-      *reinterpret_cast<uint4*>(wb + vi * VEC) = w ? ld16(w + (int64_t)vi * VEC) : make_uint4(0, 0, 0, 0);
-      *reinterpret_cast<uint4*>(wb + NMAX + vi * VEC) = b ? ld16(b + (int64_t)vi * VEC) : make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(wb + vi * VEC) = w ? RV::ld(w + rv.col(vi)) : make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(wb + NMAX + vi * VEC) = b ? RV::ld(b + rv.col(vi)) : make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
   }
@@ -84,7 +143,7 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
       const int vi = c * kWave + lane;
-      wvs[c] = (w && vi < nvec) ? ld16(w + (int64_t)vi * VEC) : make_uint4(0, 0, 0, 0);
+      wvs[c] = (w && vi < nvec) ? RV::ld(w + rv.col(vi)) : make_uint4(0, 0, 0, 0);
     }
   }
   if (RES) {
@@ -94,12 +153,12 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
     for (int c = 0; c < CHUNKS; ++c) {
       const int vi = c * kWave + lane;
       if (vi < nvec) {
-        const uint4 rv = ld16_nt(rr + (int64_t)vi * VEC);
+        const uint4 av = RV::ld_nt(rr + rv.col(vi));
         float f[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) f[e] = elem<T>(v[c], e) + elem<T>(rv, e);
+        for (int e = 0; e < VEC; ++e) f[e] = elem<T>(v[c], e) + elem<T>(av, e);
         v[c] = pack16<T>(f);
-        st16_nt(hr + (int64_t)vi * VEC, v[c]);
+        RV::st_wide(hr + rv.col(vi), v[c]);
       }
     }
   }
@@ -108,17 +167,20 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
   if (LAYER) {
     float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c)
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int dup = rv.dup(c * kWave + lane);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) s += elem<T>(v[c], e);
+      for (int e = 0; e < VEC; ++e) s += RV::counts(e, dup) ? elem<T>(v[c], e) : 0.f;
+    }
     mu = wave_sum(s) / fdim;
     float s2 = 0.f;
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
       if (c * kWave + lane < nvec) {
+        const int dup = rv.dup(c * kWave + lane);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          const float d = elem<T>(v[c], e) - mu;
+          const float d = RV::counts(e, dup) ? elem<T>(v[c], e) - mu : 0.f;
           s2 = __builtin_fmaf(d, d, s2);
         }
       }
@@ -130,12 +192,14 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
     // could contract a*a + b*b either way) give identical statistics.
     float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c)
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int dup = rv.dup(c * kWave + lane);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        const float t = elem<T>(v[c], e);
+        const float t = RV::counts(e, dup) ? elem<T>(v[c], e) : 0.f;
         s = __builtin_fmaf(t, t, s);
       }
+    }
     rstd = 1.0f / sqrtf(wave_sum(s) / fdim + eps);
   }
   T* yr = y + row * (int64_t)dim;
@@ -158,7 +222,7 @@ __global__ __launch_bounds__(fwd_threads<fwd_waves<LAYER>()>()) void norm_fwd_ve
         if (LAYER && b) t += elem<T>(bv, e);
         f[e] = t;
       }
-      st16_nt(yr + (int64_t)vi * VEC, pack16<T>(f));
+      RV::st_wide(yr + rv.col(vi), pack16<T>(f));
     }
   }
   if (lane == 0) {
@@ -236,36 +300,37 @@ constexpr int short_groups() {
   return CH == 1 ? 4 : 2;
 }
 
-template <typename T, int LPR, int CH, int G, bool LAYER, bool RES>
+template <typename T, int LPR, int CH, int G, bool LAYER, bool RES, bool ODD>
 __global__ __launch_bounds__(kFwdWaves* kWave) void norm_fwd_short(
     const T* __restrict__ x, const T* __restrict__ res, const T* __restrict__ w,
     const T* __restrict__ b, T* __restrict__ hout, T* __restrict__ y,
     float* __restrict__ mean_out, float* __restrict__ rstd_out, int64_t rows, int dim, float eps) {
   constexpr int VEC = 16 / sizeof(T), RPW = kWave / LPR;
   const int lane = threadIdx.x & (kWave - 1), l = lane % LPR;
-  const int nvec = dim / VEC;
+  typedef RowVec<T, ODD> RV;
+  const RV rv(dim);
   // consecutive waves take consecutive row groups, a workgroup G strips of them
   const int64_t first = ((int64_t)blockIdx.x * G * kFwdWaves + threadIdx.x / kWave) * RPW + lane / LPR;
-  uint4 v[G][CH], rv[RES ? G : 1][CH], wv[CH], bv[LAYER ? CH : 1];
+  uint4 v[G][CH], av[RES ? G : 1][CH], wv[CH], bv[LAYER ? CH : 1];
   bool own[CH];
 #pragma unroll
-  for (int c = 0; c < CH; ++c) own[c] = c * LPR + l < nvec;
+  for (int c = 0; c < CH; ++c) own[c] = c * LPR + l < rv.nvec;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     const int64_t row = first + g * kFwdWaves * RPW;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int64_t off = row * dim + (c * LPR + l) * VEC;
+      const int64_t off = row * dim + rv.col(c * LPR + l);
       const bool ok = own[c] && row < rows;
-      v[g][c] = ok ? ld16_nt(x + off) : make_uint4(0, 0, 0, 0);
-      if (RES) rv[g][c] = ok ? ld16_nt(res + off) : make_uint4(0, 0, 0, 0);
+      v[g][c] = ok ? RV::ld_nt(x + off) : make_uint4(0, 0, 0, 0);
+      if (RES) av[g][c] = ok ? RV::ld_nt(res + off) : make_uint4(0, 0, 0, 0);
     }
   }
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int64_t off = (c * LPR + l) * VEC;
-    wv[c] = (w && own[c]) ? ld16(w + off) : make_uint4(0, 0, 0, 0);
-    if (LAYER) bv[c] = (b && own[c]) ? ld16(b + off) : make_uint4(0, 0, 0, 0);
+    const int off = rv.col(c * LPR + l);
+    wv[c] = (w && own[c]) ? RV::ld(w + off) : make_uint4(0, 0, 0, 0);
+    if (LAYER) bv[c] = (b && own[c]) ? RV::ld(b + off) : make_uint4(0, 0, 0, 0);
   }
   const float fdim = (float)dim;
 #pragma unroll
@@ -277,26 +342,30 @@ __global__ __launch_bounds__(kFwdWaves* kWave) void norm_fwd_short(
       for (int c = 0; c < CH; ++c) {
         float f[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) f[e] = elem<T>(v[g][c], e) + elem<T>(rv[g][c], e);
+        for (int e = 0; e < VEC; ++e) f[e] = elem<T>(v[g][c], e) + elem<T>(av[g][c], e);
         v[g][c] = pack16<T>(f);
-        if (live && own[c]) st16_nt(hout + row * dim + (c * LPR + l) * VEC, v[g][c]);
+        if (live && own[c]) RV::st_nt(hout + row * dim + rv.col(c * LPR + l), v[g][c]);
       }
     }
     float mu = 0.f, s = 0.f;
     if (LAYER) {
 #pragma unroll
-      for (int c = 0; c < CH; ++c)
+      for (int c = 0; c < CH; ++c) {
+        const int dup = rv.dup(c * LPR + l);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) s += elem<T>(v[g][c], e);
+        for (int e = 0; e < VEC; ++e) s += RV::counts(e, dup) ? elem<T>(v[g][c], e) : 0.f;
+      }
       mu = group_sum<LPR>(s) / fdim;
       s = 0.f;
     }
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
       if (LAYER && !own[c]) continue;
+      const int dup = rv.dup(c * LPR + l);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        const float d = LAYER ? elem<T>(v[g][c], e) - mu : elem<T>(v[g][c], e);
+        float d = LAYER ? elem<T>(v[g][c], e) - mu : elem<T>(v[g][c], e);
+        if (!RV::counts(e, dup)) d = 0.f;
         s = __builtin_fmaf(d, d, s);
       }
     }
@@ -311,7 +380,7 @@ __global__ __launch_bounds__(kFwdWaves* kWave) void norm_fwd_short(
         if (LAYER && b) t += elem<T>(bv[c], e);
         f[e] = t;
       }
-      if (live && own[c]) st16_nt(y + row * dim + (c * LPR + l) * VEC, pack16<T>(f));
+      if (live && own[c]) RV::st_nt(y + row * dim + rv.col(c * LPR + l), pack16<T>(f));
     }
     if (live && l == 0) {
       if (rstd_out) rstd_out[row] = rstd;
@@ -394,7 +463,7 @@ constexpr int kBwdWarps = kBwdThreads / kWave;
 // One step's rows: this thread's 16-byte vectors of x, dy (and dres) for R
 // rows, with the rows' statistics.  The kernel keeps two of these and loads
 // the next step's rows while it reduces and writes the current one.
-template <typename T, int CPT, int R, int TEAM, bool LAYER, bool RES>
+template <typename T, int CPT, int R, int TEAM, bool LAYER, bool RES, bool ODD>
 struct BwdRows {
   uint4 xv[R][CPT], gv[R][CPT], hv[RES ? R : 1][CPT];
   float rs[R], mu[R];
@@ -403,8 +472,8 @@ struct BwdRows {
                                        const T* __restrict__ dres,
                                        const float* __restrict__ mean_in,
                                        const float* __restrict__ rstd_in, const bool* own,
-                                       int64_t rb, int64_t r1, int dim, int tid) {
-    constexpr int VEC = 16 / sizeof(T);
+                                       int64_t rb, int64_t r1, int dim, const int (&cols)[CPT]) {
+    typedef RowVec<T, ODD> RV;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int64_t row = rb + r;
@@ -413,10 +482,10 @@ struct BwdRows {
       mu[r] = (LAYER && ok) ? mean_in[row] : 0.f;
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
-        const int64_t off = row * (int64_t)dim + (int64_t)(tid + k * TEAM) * VEC;
-        xv[r][k] = (ok && own[k]) ? ld16_nt(x + off) : make_uint4(0, 0, 0, 0);
-        gv[r][k] = (ok && own[k]) ? ld16_nt(dy + off) : make_uint4(0, 0, 0, 0);
-        if (RES) hv[r][k] = (ok && own[k]) ? ld16_nt(dres + off) : make_uint4(0, 0, 0, 0);
+        const int64_t off = row * (int64_t)dim + cols[k];
+        xv[r][k] = (ok && own[k]) ? RV::ld_nt(x + off) : make_uint4(0, 0, 0, 0);
+        gv[r][k] = (ok && own[k]) ? RV::ld_nt(dy + off) : make_uint4(0, 0, 0, 0);
+        if (RES) hv[r][k] = (ok && own[k]) ? RV::ld_nt(dres + off) : make_uint4(0, 0, 0, 0);
       }
     }
   }
@@ -430,11 +499,12 @@ struct BwdRows {
 //   LayerNorm  dx = rstd * g - rstd*b * x-hat - rstd*a,  a = mean(g), b = mean(g * x-hat)
 //   RMSNorm    dx = rstd * g - k * x,                    k = rstd^3 * mean(g * x)
 // with g = dy * w (reference varlen_layernorm.py:64-74, varlen_rmsnorm.py:58-65).
-template <typename T, int CPT, int R, int TEAM, bool LAYER, bool RES>
-__device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, TEAM, LAYER, RES>& st,
+template <typename T, int CPT, int R, int TEAM, bool LAYER, bool RES, bool ODD>
+__device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, TEAM, LAYER, RES, ODD>& st,
                                               float (&red)[2][R][2][TEAM / kWave], int buf,
                                               const float (&wf)[CPT][16 / sizeof(T)],
-                                              const bool* own,
+                                              const bool* own, const int (&cols)[CPT],
+                                              const int (&dups)[CPT],
                                               float (&aw)[CPT][16 / sizeof(T)],
                                               float (&ab)[LAYER ? CPT : 1][16 / sizeof(T)],
                                               T* __restrict__ dx, int64_t rb, int64_t r1, int dim,
@@ -452,7 +522,8 @@ __device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, TEAM, LAYER, RE
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const float xx = elem<T>(st.xv[r][k], e);
-        const float g = elem<T>(st.gv[r][k], e) * wf[k][e];
+        float g = elem<T>(st.gv[r][k], e) * wf[k][e];
+        if (!RowVec<T, ODD>::counts(e, dups[k])) g = 0.f;
         if (LAYER) {
           s1[r] += g;
           s2[r] = fmaf(g, fmaf(xx, st.rs[r], nmr[r]), s2[r]);
@@ -518,14 +589,14 @@ __device__ __forceinline__ void norm_bwd_step(BwdRows<T, CPT, R, TEAM, LAYER, RE
         }
         if (RES) f[e] += elem<T>(st.hv[RES ? r : 0][k], e);
       }
-      st16_nt(dx + row * (int64_t)dim + (int64_t)(tid + k * TEAM) * VEC, pack16<T>(f));
+      RowVec<T, ODD>::st_wide(dx + row * (int64_t)dim + cols[k], pack16<T>(f));
     }
   }
 }
 
 // RES: dx also receives dres (the gradient reaching the normalised input by
 // another path, e.g. the residual stream of an add + RMSNorm).
-template <typename T, int CPT, int R, int TW, int TEAMS, bool LAYER, bool RES>
+template <typename T, int CPT, int R, int TW, int TEAMS, bool LAYER, bool RES, bool ODD>
 __global__ __launch_bounds__(TW* TEAMS* kWave) void norm_bwd_cols(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ mean_in, const float* __restrict__ rstd_in,
@@ -537,15 +608,19 @@ __global__ __launch_bounds__(TW* TEAMS* kWave) void norm_bwd_cols(
   // (a team is whole waves: its index, and with it every row's address, is scalar)
   const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / TEAM) : 0;
   const int tid = (int)threadIdx.x - team * TEAM;
-  const int nvec = dim / VEC;
+  typedef RowVec<T, ODD> RV;
+  const RV rv(dim);
 
   float wf[CPT][VEC];  // this thread's weights as fp32, ones without a weight
   bool own[CPT];
+  int cols[CPT], dups[CPT];  // first column of each vector, and its repeated elements (ODD)
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int v = tid + k * TEAM;
-    own[k] = v < nvec;
-    const uint4 wv = (w && own[k]) ? ld16(w + (int64_t)v * VEC) : make_uint4(0, 0, 0, 0);
+    own[k] = v < rv.nvec;
+    cols[k] = rv.col(v);
+    dups[k] = rv.dup(v);
+    const uint4 wv = (w && own[k]) ? RV::ld(w + cols[k]) : make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) wf[k][e] = w ? elem<T>(wv, e) : 1.0f;
   }
@@ -561,20 +636,20 @@ __global__ __launch_bounds__(TW* TEAMS* kWave) void norm_bwd_cols(
   // Two row sets: while one step reduces and writes, the next step's rows
   // load.  Steps are S rows apart; rows past the end load as zeros and are
   // not written.
-  BwdRows<T, CPT, R, TEAM, LAYER, RES> A, B;
+  BwdRows<T, CPT, R, TEAM, LAYER, RES, ODD> A, B;
   const float inv_dim = 1.0f / (float)dim;
   // (with several teams every one runs the block's count of steps: they share
   // the steps' barriers; rows past the end load as zeros)
   const int64_t S = (int64_t)gridDim.x * TEAMS * R;
   const int64_t lead = (int64_t)blockIdx.x * TEAMS * R;  // the block's first row
   const int64_t first = lead + team * R, lag = first - lead;
-  if (lead < rows) A.load(x, dy, dres, mean_in, rstd_in, own, first, rows, dim, tid);
+  if (lead < rows) A.load(x, dy, dres, mean_in, rstd_in, own, first, rows, dim, cols);
   for (int64_t rb = first; rb - lag < rows; rb += 2 * S) {
-    if (rb - lag + S < rows) B.load(x, dy, dres, mean_in, rstd_in, own, rb + S, rows, dim, tid);
-    norm_bwd_step<T, CPT, R, TEAM, LAYER, RES>(A, red[team], 0, wf, own, aw, ab, dx, rb, rows, dim, inv_dim, tid);
+    if (rb - lag + S < rows) B.load(x, dy, dres, mean_in, rstd_in, own, rb + S, rows, dim, cols);
+    norm_bwd_step<T, CPT, R, TEAM, LAYER, RES, ODD>(A, red[team], 0, wf, own, cols, dups, aw, ab, dx, rb, rows, dim, inv_dim, tid);
     if (rb - lag + S >= rows) break;
-    if (rb - lag + 2 * S < rows) A.load(x, dy, dres, mean_in, rstd_in, own, rb + 2 * S, rows, dim, tid);
-    norm_bwd_step<T, CPT, R, TEAM, LAYER, RES>(B, red[team], 1, wf, own, aw, ab, dx, rb + S, rows, dim, inv_dim, tid);
+    if (rb - lag + 2 * S < rows) A.load(x, dy, dres, mean_in, rstd_in, own, rb + 2 * S, rows, dim, cols);
+    norm_bwd_step<T, CPT, R, TEAM, LAYER, RES, ODD>(B, red[team], 1, wf, own, cols, dups, aw, ab, dx, rb + S, rows, dim, inv_dim, tid);
   }
   __shared__ __align__(16) float tsum[TEAMS > 1 ? TEAMS - 1 : 1][TEAMS > 1 ? CPT * TEAM * VEC : 1];
   auto write = [&](int p, auto& acc) {
@@ -599,7 +674,13 @@ __global__ __launch_bounds__(TW* TEAMS* kWave) void norm_bwd_cols(
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       if (!own[k]) continue;
-      float* o = out + (int64_t)(tid + k * TEAM) * VEC;
+      float* o = out + cols[k];
+      if constexpr (ODD) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          if (RV::counts(e, dups[k])) o[e] = acc[k][e];
+        continue;
+      }
 #pragma unroll
       for (int e = 0; e < VEC; e += 4)
         *reinterpret_cast<float4*>(o + e) = make_float4(acc[k][e], acc[k][e + 1], acc[k][e + 2], acc[k][e + 3]);
@@ -617,7 +698,7 @@ __global__ __launch_bounds__(TW* TEAMS* kWave) void norm_bwd_cols(
 // order, into the block's partial row.  Blocks take interleaved row groups as
 // in norm_bwd_cols; the next group loads during the current one where both fit
 // 128 registers (CH == 1), else four waves per SIMD cover the loads.
-template <typename T, int LPR, int CH, bool LAYER, bool RES>
+template <typename T, int LPR, int CH, bool LAYER, bool RES, bool ODD>
 struct ShortRows {
   uint4 xv[CH], gv[CH], hv[CH];
   float rs, mu;
@@ -625,17 +706,17 @@ struct ShortRows {
                                        const T* __restrict__ dres,
                                        const float* __restrict__ mean_in,
                                        const float* __restrict__ rstd_in, const bool (&own)[CH],
-                                       int64_t row, int64_t rows, int dim, int l) {
-    constexpr int VEC = 16 / sizeof(T);
+                                       int64_t row, int64_t rows, const RowVec<T, ODD>& rv, int l) {
+    typedef RowVec<T, ODD> RV;
     const bool ok = row < rows;
     rs = ok ? rstd_in[row] : 0.f;
     mu = (LAYER && ok) ? mean_in[row] : 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int64_t off = row * dim + (c * LPR + l) * VEC;
-      xv[c] = (ok && own[c]) ? ld16_nt(x + off) : make_uint4(0, 0, 0, 0);
-      gv[c] = (ok && own[c]) ? ld16_nt(dy + off) : make_uint4(0, 0, 0, 0);
-      if (RES) hv[c] = (ok && own[c]) ? ld16_nt(dres + off) : make_uint4(0, 0, 0, 0);
+      const int64_t off = row * rv.dim + rv.col(c * LPR + l);
+      xv[c] = (ok && own[c]) ? RV::ld_nt(x + off) : make_uint4(0, 0, 0, 0);
+      gv[c] = (ok && own[c]) ? RV::ld_nt(dy + off) : make_uint4(0, 0, 0, 0);
+      if (RES) hv[c] = (ok && own[c]) ? RV::ld_nt(dres + off) : make_uint4(0, 0, 0, 0);
     }
   }
 };
@@ -645,22 +726,24 @@ __device__ __forceinline__ void repack(uint4& v) {
   asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
 }
 // One step's rows; arithmetic per row as in norm_bwd_step.
-template <typename T, int LPR, int CH, bool LAYER, bool RES>
+template <typename T, int LPR, int CH, bool LAYER, bool RES, bool ODD>
 __device__ __forceinline__ void norm_bwd_short_step(
-    ShortRows<T, LPR, CH, LAYER, RES>& st, uint4 (&wv)[CH], bool has_w, const bool (&own)[CH],
+    ShortRows<T, LPR, CH, LAYER, RES, ODD>& st, uint4 (&wv)[CH], bool has_w, const bool (&own)[CH],
     float (&aw)[CH][16 / sizeof(T)], float (&ab)[LAYER ? CH : 1][16 / sizeof(T)],
-    T* __restrict__ dx, int64_t row, int64_t rows, int dim, float inv_dim, int l) {
+    T* __restrict__ dx, int64_t row, int64_t rows, const RowVec<T, ODD>& rv, float inv_dim, int l) {
   constexpr int VEC = 16 / sizeof(T);
   const float rr = st.rs, nmr = -st.mu * rr;
   float s1 = 0.f, s2 = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     repack(wv[c]);
+    const int dup = rv.dup(c * LPR + l);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       const float xx = elem<T>(st.xv[c], e);
       const float d = elem<T>(st.gv[c], e);
-      const float g = has_w ? d * elem<T>(wv[c], e) : d;
+      float g = has_w ? d * elem<T>(wv[c], e) : d;
+      if (!RowVec<T, ODD>::counts(e, dup)) g = 0.f;
       if (LAYER) {
         s1 += g;
         s2 = fmaf(g, fmaf(xx, rr, nmr), s2);
@@ -695,10 +778,10 @@ __device__ __forceinline__ void norm_bwd_short_step(
       }
       if (RES) f[e] += elem<T>(st.hv[c], e);
     }
-    if (row < rows && own[c]) st16_nt(dx + row * dim + (c * LPR + l) * VEC, pack16<T>(f));
+    if (row < rows && own[c]) RowVec<T, ODD>::st_nt(dx + row * rv.dim + rv.col(c * LPR + l), pack16<T>(f));
   }
 }
-template <typename T, int LPR, int CH, bool LAYER, bool RES>
+template <typename T, int LPR, int CH, bool LAYER, bool RES, bool ODD>
 __global__ __launch_bounds__(kBwdThreads, 4) void norm_bwd_short(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ mean_in, const float* __restrict__ rstd_in,
@@ -708,13 +791,14 @@ __global__ __launch_bounds__(kBwdThreads, 4) void norm_bwd_short(
   constexpr int RPB = kBwdWarps * RPW;  // rows of the block per step
   __shared__ __align__(16) float sums[kBwdWarps][LPR * CH * VEC];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, l = lane % LPR;
-  const int nvec = dim / VEC;
+  typedef RowVec<T, ODD> RV;
+  const RV rv(dim);
   bool own[CH];
   uint4 wv[CH];
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    own[c] = c * LPR + l < nvec;
-    wv[c] = (w && own[c]) ? ld16(w + (c * LPR + l) * VEC) : make_uint4(0, 0, 0, 0);
+    own[c] = c * LPR + l < rv.nvec;
+    wv[c] = (w && own[c]) ? RV::ld(w + rv.col(c * LPR + l)) : make_uint4(0, 0, 0, 0);
   }
   float aw[CH][VEC], ab[LAYER ? CH : 1][VEC];
 #pragma unroll
@@ -727,17 +811,17 @@ __global__ __launch_bounds__(kBwdThreads, 4) void norm_bwd_short(
   const float inv_dim = 1.0f / (float)dim;
   const int64_t S = (int64_t)gridDim.x * RPB;
   int64_t row = (int64_t)blockIdx.x * RPB + wave * RPW + lane / LPR;
-  ShortRows<T, LPR, CH, LAYER, RES> A;
-  auto load = [&](ShortRows<T, LPR, CH, LAYER, RES>& st, int64_t r) {
-    st.load(x, dy, dres, mean_in, rstd_in, own, r, rows, dim, l);
+  ShortRows<T, LPR, CH, LAYER, RES, ODD> A;
+  auto load = [&](ShortRows<T, LPR, CH, LAYER, RES, ODD>& st, int64_t r) {
+    st.load(x, dy, dres, mean_in, rstd_in, own, r, rows, rv, l);
   };
-  auto step = [&](ShortRows<T, LPR, CH, LAYER, RES>& st, int64_t r) {
-    norm_bwd_short_step<T, LPR, CH, LAYER, RES>(st, wv, w != nullptr, own, aw, ab, dx, r, rows, dim,
+  auto step = [&](ShortRows<T, LPR, CH, LAYER, RES, ODD>& st, int64_t r) {
+    norm_bwd_short_step<T, LPR, CH, LAYER, RES, ODD>(st, wv, w != nullptr, own, aw, ab, dx, r, rows, rv,
                                                 inv_dim, l);
   };
   // (the loops' condition is uniform over the wave: its first row)
   if constexpr (CH == 1) {
-    ShortRows<T, LPR, CH, LAYER, RES> B;
+    ShortRows<T, LPR, CH, LAYER, RES, ODD> B;
     load(A, row);
     for (; row - lane / LPR < rows; row += 2 * S) {
       load(B, row + S);
@@ -759,7 +843,8 @@ __global__ __launch_bounds__(kBwdThreads, 4) void norm_bwd_short(
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const float t = subgroups_sum<LPR>(acc[c][e]);
-        if (lane < LPR) sums[wave][(c * LPR + l) * VEC + e] = t;
+        const int v = c * LPR + l;
+        if (lane < LPR && v < rv.nvec && RV::counts(e, rv.dup(v))) sums[wave][rv.col(v) + e] = t;
       }
     __syncthreads();
     float* out = partial + ((int64_t)blockIdx.x * nparam + p) * dim;
@@ -847,33 +932,40 @@ __global__ __launch_bounds__(256) void norm_bwd_param_generic(
   if (nparam > 1) out[dim + col] = ab;
 }
 
-// Column sums of the partial rows; output cast to out_dtype.  Scalar form
-// (any dim): 64 columns x 4 row groups per block.
+// Column sums of the partial rows; output cast to out_dtype.
 __device__ __forceinline__ void store_param(void* out, int col, float t, int out_dtype) {
   if (out_dtype == SCREE_DTYPE_F32) static_cast<float*>(out)[col] = t;
   else if (out_dtype == SCREE_DTYPE_F16) static_cast<f16*>(out)[col] = (f16)t;
   else static_cast<bf16*>(out)[col] = (bf16)t;
 }
 
+// Any dim: 16 columns x 16 row groups per block, every load in flight at once,
+// then a fixed-order tree over the row groups in LDS.
 __global__ __launch_bounds__(256) void norm_param_colsum(const float* __restrict__ partial,
                                                          int nparts, int nparam, int dim,
                                                          void* out0, void* out1, int out_dtype) {
-  __shared__ float red[4][kWave];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int grp = threadIdx.x / kWave;
-  const int col = blockIdx.x * kWave + lane;
+  __shared__ float red[16][16];
+  const int cq = threadIdx.x & 15, rg = threadIdx.x >> 4;
+  const int col = blockIdx.x * 16 + cq;
   const int p = blockIdx.y;
-  float s = 0.f;
-  if (col < dim) {
-    for (int i = grp; i < nparts; i += 4) s += partial[((int64_t)i * nparam + p) * dim + col];
+  constexpr int kIt = kMaxParts / 16;
+  float v[kIt];
+#pragma unroll
+  for (int j = 0; j < kIt; ++j) {
+    const int i = rg + 16 * j;
+    v[j] = (col < dim && i < nparts) ? partial[((int64_t)i * nparam + p) * dim + col] : 0.f;
   }
-  red[grp][lane] = s;
+  float s = v[0];
+#pragma unroll
+  for (int j = 1; j < kIt; ++j) s += v[j];
+  red[rg][cq] = s;
   __syncthreads();
-  if (grp == 0 && col < dim) {
-    const float t = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
-    void* out = p == 0 ? out0 : out1;
-    if (out) store_param(out, col, t, out_dtype);
+  for (int st = 8; st >= 1; st >>= 1) {
+    if (rg < st) red[rg][cq] += red[rg + st][cq];
+    __syncthreads();
   }
+  void* out = p == 0 ? out0 : out1;
+  if (rg == 0 && col < dim && out) store_param(out, col, red[0][cq], out_dtype);
 }
 
 // Vector form (dim % 4 == 0): 16 columns x 64 row groups per block, 16-byte
@@ -944,26 +1036,21 @@ inline int nparts_for(int64_t rows) {
   return (int)p;
 }
 
+// How the vector kernels take rows of `dim` columns in these buffers: not at
+// all (rows shorter than a vector, or of more than max_vecs), as whole aligned
+// vectors, or as ODD ones.
+enum class RowForm { kNone, kAligned, kOdd };
 template <typename T>
-bool fast_path_ok(int64_t dim, std::initializer_list<const void*> ptrs) {
+RowForm row_form(int64_t dim, int64_t max_vecs, std::initializer_list<const void*> ptrs) {
   constexpr int VEC = 16 / sizeof(T);
-  if (dim % VEC) return false;
-  if (dim / VEC > (int64_t)kMaxChunks * kWave) return false;
+  if (dim < VEC || (dim + VEC - 1) / VEC > max_vecs) return RowForm::kNone;
+  if (dim % VEC) return RowForm::kOdd;
   for (const void* p : ptrs)
-    if (p && !aligned16(p)) return false;
-  return true;
+    if (p && !aligned16(p)) return RowForm::kOdd;
+  return RowForm::kAligned;
 }
-
-// Backward fast path: whole 16-byte vectors, at most 2 per thread of a 512-thread block.
-template <typename T>
-bool bwd_fast_path_ok(int64_t dim, std::initializer_list<const void*> ptrs) {
-  constexpr int VEC = 16 / sizeof(T);
-  if (dim % VEC) return false;
-  if (dim / VEC > 2 * (int64_t)kBwdThreads) return false;
-  for (const void* p : ptrs)
-    if (p && !aligned16(p)) return false;
-  return true;
-}
+constexpr int64_t kMaxFwdVecs = (int64_t)kMaxChunks * kWave;
+constexpr int64_t kMaxBwdVecs = 2 * (int64_t)kBwdThreads;  // two per thread of a 512-thread block
 
 // Lanes per row and vectors per lane of the short-row kernels: the pair that
 // covers nvec vectors with the fewest idle lanes, {0, 0} past their range.
@@ -987,20 +1074,20 @@ inline ShortShape short_shape(int64_t nvec, bool thirds) {
   CASE(32, 3)                   \
   CASE(64, 2)
 
-// res / h non-null (RMSNorm only): normalise h = x + res and write h too.
-template <typename T, bool LAYER, bool RES>
-void launch_fwd_k(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* yp, float* mean,
-                  float* rstd, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
-  const dim3 grid((unsigned)((rows + kFwdWaves - 1) / kFwdWaves));
+// The vector kernels (rows of whole 16-byte vectors, or ODD).
+template <typename T, bool LAYER, bool RES, bool ODD>
+void launch_fwd_vec(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* yp, float* mean,
+                    float* rstd, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
   const dim3 block(kFwdWaves * kWave);
   const int d = (int)dim;
-  if (fast_path_ok<T>(dim, {xp, rp, wp, bp, hp, yp})) {
-    const ShortShape sh = short_shape(dim / (16 / (int64_t)sizeof(T)), true);
-    if (sh.ch) {
+  constexpr int64_t VEC = 16 / sizeof(T);
+  const int64_t nvec = (dim + VEC - 1) / VEC;
+  const ShortShape sh = short_shape(nvec, true);
+  if (sh.ch) {
 #define SCREE_FWD_SHORT_G(L, C, G)                                                                 \
-  hipLaunchKernelGGL((norm_fwd_short<T, L, C, G, LAYER, RES>),                                     \
-                     dim3((unsigned)((rows + per * G - 1) / (per * G))), block, 0, stream, xp, rp, \
-                     wp, bp, hp, yp, mean, rstd, rows, d, eps)
+  hipLaunchKernelGGL((norm_fwd_short<T, L, C, G, LAYER, RES, ODD>),                                     \
+                   dim3((unsigned)((rows + per * G - 1) / (per * G))), block, 0, stream, xp, rp, \
+                   wp, bp, hp, yp, mean, rstd, rows, d, eps)
 #define SCREE_FWD_SHORT(L, C)                                                                      \
   if (sh.lpr == L && sh.ch == C) {                                                                 \
     constexpr int64_t per = (int64_t)kFwdWaves * (kWave / L);                                      \
@@ -1010,29 +1097,41 @@ void launch_fwd_k(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* 
       SCREE_FWD_SHORT_G(L, C, 1);                                                                  \
     return;                                                                                        \
   }
-      SCREE_SHORT_CASES(SCREE_FWD_SHORT)
+    SCREE_SHORT_CASES(SCREE_FWD_SHORT)
 #undef SCREE_FWD_SHORT
 #undef SCREE_FWD_SHORT_G
-    }
-    constexpr int W = fwd_waves<LAYER>();
-    const dim3 vgrid((unsigned)((rows + W - 1) / W)), vblock(W * kWave);
-    const int chunks = chunks_for((int)(dim / (16 / sizeof(T))));
+  }
+  constexpr int W = fwd_waves<LAYER>();
+  const dim3 vgrid((unsigned)((rows + W - 1) / W)), vblock(W * kWave);
+  const int chunks = chunks_for((int)nvec);
 #define SCREE_FWD_CASE(C)                                                                      \
   case C:                                                                                      \
-    hipLaunchKernelGGL((norm_fwd_vec<T, C, LAYER, RES>), vgrid, vblock, 0, stream, xp, rp, wp, bp, \
-                       hp, yp, mean, rstd, rows, d, eps);                                      \
-    break;
-    switch (chunks) {
-      SCREE_FWD_CASE(4)
-      SCREE_FWD_CASE(8)
-      SCREE_FWD_CASE(16)
-      default: break;  // chunks_for never exceeds kMaxChunks on the fast path
-    }
-#undef SCREE_FWD_CASE
-  } else {
-    hipLaunchKernelGGL((norm_fwd_generic<T, LAYER, RES>), grid, block, 0, stream, xp, rp, wp, bp,
-                       hp, yp, mean, rstd, rows, d, eps);
+  hipLaunchKernelGGL((norm_fwd_vec<T, C, LAYER, RES, ODD>), vgrid, vblock, 0, stream, xp, rp, wp, bp, \
+                     hp, yp, mean, rstd, rows, d, eps);                                      \
+  break;
+  switch (chunks) {
+    SCREE_FWD_CASE(4)
+    SCREE_FWD_CASE(8)
+    SCREE_FWD_CASE(16)
+    default: break;  // chunks_for never exceeds kMaxChunks on the fast path
   }
+#undef SCREE_FWD_CASE
+}
+
+// res / h non-null (RMSNorm only): normalise h = x + res and write h too.
+template <typename T, bool LAYER, bool RES>
+void launch_fwd_k(const T* xp, const T* rp, const T* wp, const T* bp, T* hp, T* yp, float* mean,
+                  float* rstd, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
+  switch (row_form<T>(dim, kMaxFwdVecs, {xp, rp, wp, bp, hp, yp})) {
+    case RowForm::kAligned:
+      return launch_fwd_vec<T, LAYER, RES, false>(xp, rp, wp, bp, hp, yp, mean, rstd, rows, dim, eps, stream);
+    case RowForm::kOdd:
+      return launch_fwd_vec<T, LAYER, RES, true>(xp, rp, wp, bp, hp, yp, mean, rstd, rows, dim, eps, stream);
+    case RowForm::kNone: break;
+  }
+  const dim3 grid((unsigned)((rows + kFwdWaves - 1) / kFwdWaves)), block(kFwdWaves * kWave);
+  hipLaunchKernelGGL((norm_fwd_generic<T, LAYER, RES>), grid, block, 0, stream, xp, rp, wp, bp, hp, yp,
+                     mean, rstd, rows, (int)dim, eps);
 }
 
 template <typename T, bool LAYER>
@@ -1056,62 +1155,79 @@ int launch_fwd(const void* x, const void* res, const void* w, const void* b, voi
   return check_launch(LAYER ? "scree_layernorm_fwd" : "scree_rmsnorm_fwd");
 }
 
+// The vector kernels (rows of whole 16-byte vectors, or ODD); returns the
+// number of partial rows written, at most `nparts`.
+template <typename T, bool LAYER, bool RES, bool ODD>
+int launch_bwd_vec(const T* dyp, const T* xp, const T* wp, const float* mean, const float* rstd,
+                   const T* dresp, T* dxp, float* partial, bool want_params, int nparts,
+                   int64_t rows, int64_t dim, hipStream_t stream) {
+  const int d = (int)dim;
+  const int nparam = LAYER ? 2 : 1;
+  constexpr int VEC = 16 / sizeof(T);
+  const int nvec = (int)((dim + VEC - 1) / VEC);
+  const int cpt = (nvec + kBwdThreads - 1) / kBwdThreads;  // 1 or 2
+  const dim3 grid((unsigned)nparts), block(kBwdThreads);
+  const int np = want_params ? nparam : 0;
+  // (three vectors per lane would spill with two sums each, or as ODD ones with a residual)
+  constexpr bool kThirds = !LAYER && !(RES && ODD);
+  const ShortShape sh = short_shape(nvec, kThirds);
+  if (sh.ch) {
+#define SCREE_BWD_SHORT(L, C)                                                                       \
+  if constexpr (C != 3 || kThirds) {                                                                \
+    if (sh.lpr == L && sh.ch == C) {                                                                \
+      constexpr int64_t per = (int64_t)kBwdWarps * (kWave / L);                                     \
+      nparts = (int)std::min<int64_t>(nparts, std::max<int64_t>(1, (rows + per - 1) / per));        \
+      hipLaunchKernelGGL((norm_bwd_short<T, L, C, LAYER, RES, ODD>), dim3((unsigned)nparts), block, \
+                         0, stream, dyp, xp, wp, mean, rstd, dresp, dxp, partial, rows, d, np);     \
+      return nparts;                                                                                \
+    }                                                                                               \
+  }
+    SCREE_SHORT_CASES(SCREE_BWD_SHORT)
+#undef SCREE_BWD_SHORT
+  }
+  // rows per step: two steps' rows (double-buffered) fit 4 waves per SIMD
+  // (LN keeps two sums per row; the residual gradient is one more vector).
+  // At one vector per thread 2 rows per step measured best for all three
+  // (RMSNorm at config 2: R = 1, 2, 3, 4 -> 90.8, 87.3, 89.1, 90.5 us).
+  constexpr int R1 = 2;
+  constexpr int R2 = (LAYER || RES) ? 1 : 2;
+#define SCREE_BWD_COLS(CPT, R, TW, TEAMS)                                                          \
+  hipLaunchKernelGGL((norm_bwd_cols<T, CPT, R, TW, TEAMS, LAYER, RES, ODD>), grid,                      \
+                   dim3(TW * TEAMS * kWave), 0, stream, dyp, xp, wp, mean, rstd, dresp, dxp,     \
+                   partial, rows, d, np)
+  if (nvec <= 3 * kWave)
+    SCREE_BWD_COLS(1, R1, 3, 2);
+  else if (nvec <= 4 * kWave)
+    SCREE_BWD_COLS(1, R1, 4, 2);
+  else if (cpt == 1)
+    SCREE_BWD_COLS(1, R1, kBwdWarps, 1);
+  else
+    SCREE_BWD_COLS(2, R2, kBwdWarps, 1);
+#undef SCREE_BWD_COLS
+  return nparts;
+}
+
 // dres non-null (RMSNorm only): dx also receives dres.  Returns the number of
 // partial rows written, at most `nparts`.
 template <typename T, bool LAYER, bool RES>
 int launch_bwd_k(const T* dyp, const T* xp, const T* wp, const float* mean, const float* rstd,
-                  const T* dresp, T* dxp, float* partial, bool want_params, int nparts,
-                  int64_t rows, int64_t dim, hipStream_t stream) {
+                 const T* dresp, T* dxp, float* partial, bool want_params, int nparts,
+                 int64_t rows, int64_t dim, hipStream_t stream) {
+  switch (row_form<T>(dim, kMaxBwdVecs, {dyp, xp, wp, dresp, dxp})) {
+    case RowForm::kAligned: return launch_bwd_vec<T, LAYER, RES, false>(dyp, xp, wp, mean, rstd, dresp, dxp, partial, want_params, nparts, rows, dim, stream);
+    case RowForm::kOdd: return launch_bwd_vec<T, LAYER, RES, true>(dyp, xp, wp, mean, rstd, dresp, dxp, partial, want_params, nparts, rows, dim, stream);
+    case RowForm::kNone: break;
+  }
   const int d = (int)dim;
   const int nparam = LAYER ? 2 : 1;
-  if (bwd_fast_path_ok<T>(dim, {dyp, xp, wp, dresp, dxp})) {
-    const int nvec = (int)(dim / (16 / sizeof(T)));
-    const int cpt = (nvec + kBwdThreads - 1) / kBwdThreads;  // 1 or 2
-    const dim3 grid((unsigned)nparts), block(kBwdThreads);
-    const int np = want_params ? nparam : 0;
-    // (three vectors per lane with two sums each would spill)
-    const ShortShape sh = short_shape(nvec, !LAYER);
-    if (sh.ch) {
-#define SCREE_BWD_SHORT(L, C)                                                                       \
-  if (sh.lpr == L && sh.ch == C) {                                                                  \
-    constexpr int64_t per = (int64_t)kBwdWarps * (kWave / L);          \
-    nparts = (int)std::min<int64_t>(nparts, std::max<int64_t>(1, (rows + per - 1) / per));          \
-    hipLaunchKernelGGL((norm_bwd_short<T, L, C, LAYER, RES>), dim3((unsigned)nparts), block, 0,     \
-                       stream, dyp, xp, wp, mean, rstd, dresp, dxp, partial, rows, d, np);          \
-    return nparts;                                                                                  \
-  }
-      SCREE_SHORT_CASES(SCREE_BWD_SHORT)
-#undef SCREE_BWD_SHORT
-    }
-    // rows per step: two steps' rows (double-buffered) fit 4 waves per SIMD
-    // (LN keeps two sums per row; the residual gradient is one more vector).
-    // At one vector per thread 2 rows per step measured best for all three
-    // (RMSNorm at config 2: R = 1, 2, 3, 4 -> 90.8, 87.3, 89.1, 90.5 us).
-    constexpr int R1 = 2;
-    constexpr int R2 = (LAYER || RES) ? 1 : 2;
-#define SCREE_BWD_COLS(CPT, R, TW, TEAMS)                                                          \
-  hipLaunchKernelGGL((norm_bwd_cols<T, CPT, R, TW, TEAMS, LAYER, RES>), grid,                      \
-                     dim3(TW * TEAMS * kWave), 0, stream, dyp, xp, wp, mean, rstd, dresp, dxp,     \
-                     partial, rows, d, np)
-    if (nvec <= 3 * kWave)
-      SCREE_BWD_COLS(1, R1, 3, 2);
-    else if (nvec <= 4 * kWave)
-      SCREE_BWD_COLS(1, R1, 4, 2);
-    else if (cpt == 1)
-      SCREE_BWD_COLS(1, R1, kBwdWarps, 1);
-    else
-      SCREE_BWD_COLS(2, R2, kBwdWarps, 1);
-#undef SCREE_BWD_COLS
-  } else {
-    const dim3 grid((unsigned)((rows + kFwdWaves - 1) / kFwdWaves)), block(kFwdWaves * kWave);
-    if (rows > 0)
-      hipLaunchKernelGGL((norm_bwd_dx_generic<T, LAYER, RES>), grid, block, 0, stream, dyp, xp, wp,
-                         mean, rstd, dresp, dxp, rows, d);
-    if (want_params) {
-      const dim3 pgrid((unsigned)((dim + 255) / 256), (unsigned)nparts);
-      hipLaunchKernelGGL((norm_bwd_param_generic<T, LAYER>), pgrid, dim3(256), 0, stream, dyp, xp,
-                         mean, rstd, partial, rows, d, nparam);
-    }
+  const dim3 grid((unsigned)((rows + kFwdWaves - 1) / kFwdWaves)), block(kFwdWaves * kWave);
+  if (rows > 0)
+    hipLaunchKernelGGL((norm_bwd_dx_generic<T, LAYER, RES>), grid, block, 0, stream, dyp, xp, wp,
+                       mean, rstd, dresp, dxp, rows, d);
+  if (want_params) {
+    const dim3 pgrid((unsigned)((dim + 255) / 256), (unsigned)nparts);
+    hipLaunchKernelGGL((norm_bwd_param_generic<T, LAYER>), pgrid, dim3(256), 0, stream, dyp, xp,
+                       mean, rstd, partial, rows, d, nparam);
   }
   return nparts;
 }
@@ -1149,7 +1265,7 @@ int launch_bwd(const void* dy, const void* x, const void* w, const float* mean, 
     hipLaunchKernelGGL(norm_param_colsum4, cgrid, dim3(256), 0, stream, partial, nparts, nparam, d,
                        dw, db, dparam_dtype);
   } else {
-    const dim3 cgrid((unsigned)((dim + kWave - 1) / kWave), (unsigned)nparam);
+    const dim3 cgrid((unsigned)((dim + 15) / 16), (unsigned)nparam);
     hipLaunchKernelGGL(norm_param_colsum, cgrid, dim3(256), 0, stream, partial, nparts, nparam, d,
                        dw, db, dparam_dtype);
   }
