@@ -692,19 +692,19 @@ constexpr int acc_row0(int i) { return 8 * (i >> 2) + (i & 3); }
 // the block loop.  The forward (OPAQUE = false) masks only in the blocks of
 // its peeled diagonal loop, where the plain form needs no extra register.
 template <bool OPAQUE = true>
-__device__ __forceinline__ void mask_rows_above(f32x16& c, int rel_minus_4g) {
+__device__ __forceinline__ void mask_rows_above(f32x16& c, int rel_minus_4g, float fill = kNegInf) {
   if (OPAQUE) asm volatile("" : "+v"(rel_minus_4g));
 #pragma unroll
   for (int i = 0; i < 16; ++i)
-    if (acc_row0(i) > rel_minus_4g) c[i] = kNegInf;
+    if (acc_row0(i) > rel_minus_4g) c[i] = fill;
 }
 // The converse: mask the elements whose row is below `rel` (acc_row0(i) <
 // rel - 4g).
-__device__ __forceinline__ void mask_rows_below(f32x16& c, int rel_minus_4g) {
+__device__ __forceinline__ void mask_rows_below(f32x16& c, int rel_minus_4g, float fill = kNegInf) {
   asm volatile("" : "+v"(rel_minus_4g));
 #pragma unroll
   for (int i = 0; i < 16; ++i)
-    if (acc_row0(i) < rel_minus_4g) c[i] = kNegInf;
+    if (acc_row0(i) < rel_minus_4g) c[i] = fill;
 }
 
 // Wave index as a scalar, so per-wave tile bounds are uniform branches.
@@ -2718,13 +2718,14 @@ __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dq_f32m_
       __builtin_amdgcn_sched_barrier(0);
       if (more) tv.rows(Y, vh, 32 * (kt + KG), L);
       __builtin_amdgcn_sched_barrier(0);
-      if (CAUSAL) {
-        if (32 * kt == qw0) mask_rows_above<false>(s, r - 4 * g);
-      } else if (32 * kt + 32 > L) {
-        mask_rows_above<false>(s, L - 1 - 32 * kt - 4 * g);
-      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = fast_exp2(fmaf(s[i], c, -lse2)) * (dp[i] - dl);
+      // (dS is masked, not the scores: -inf times a scale of 0 or less gives no weight of 0)
+      if (CAUSAL) {
+        if (32 * kt == qw0) mask_rows_above<false>(s, r - 4 * g, 0.f);
+      } else if (32 * kt + 32 > L) {
+        mask_rows_above<false>(s, L - 1 - 32 * kt - 4 * g, 0.f);
+      }
       f32m_accum<D>(dqacc, 1.0f, Z, s);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -2845,8 +2846,6 @@ __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dkv_f32m
       __builtin_amdgcn_sched_barrier(0);
       tq.cols(Y, cqh, cur, L);
       __builtin_amdgcn_sched_barrier(0);
-      if (CAUSAL && cur == kw0) mask_rows_below(s, r - 4 * g);  // queries before the key
-      if (cur + 32 > L) mask_rows_above(s, L - 1 - cur - 4 * g);
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // this wave's own row statistics
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
@@ -2857,9 +2856,14 @@ __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dkv_f32m
         for (int e = 0; e < 4; ++e) {
           const int i = 4 * i4 + e;
           s[i] = fast_exp2(fmaf(s[i], c, -la[e]));
-          dp[i] = s[i] * (dp[i] - da[e]);
+          dp[i] -= da[e];
         }
       }
+      // (the weights are masked, not the scores, as in dQ)
+      if (CAUSAL && cur == kw0) mask_rows_below(s, r - 4 * g, 0.f);  // queries before the key
+      if (cur + 32 > L) mask_rows_above(s, L - 1 - cur - 4 * g, 0.f);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dp[i] *= s[i];
       f32m_accum<D>(dvacc, 1.0f, X, s);
       __builtin_amdgcn_sched_barrier(0);
       if (more) tq.rows(X, qh, qb, L);

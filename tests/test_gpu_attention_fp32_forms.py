@@ -52,3 +52,49 @@ def test_fp32_single_token_any_row_stride(dim):
     assert torch.equal(got[0], base[2])  # the only key's value
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def _c_abi_step(q, k, v, do, cu, causal, scale):
+    """Forward and backward through the C entry points, which take any scale."""
+    from scree_amd.kernels.hip import _ffi
+    from scree_amd.kernels.hip import attention as A
+
+    lib, (n, heads, dim) = _ffi.lib(), q.shape
+    o, dq, dk, dv = (torch.empty_like(t) for t in (q, q, k, v))
+    lse = torch.empty((n, heads), device=q.device)
+    delta = torch.empty_like(lse)
+    ws = A.attention_schedule(cu, n, dim, causal)
+
+    def call(fn, ts, strided):
+        strides = _ffi.int64_array(sum((t.stride()[:2] for t in strided), ()))
+        _ffi.check(fn(*map(_ffi.ptr, ts), _ffi.ptr(cu), cu.numel() - 1, n, heads, k.shape[1], dim,
+                      strides, scale, int(causal), _ffi.DTYPE_F32, _ffi.ptr(ws), ws.numel(),
+                      _ffi.stream_of(q)))
+
+    call(lib.scree_attn_fwd_gqa, (q, k, v, o, lse), (q, k, v, o))
+    call(lib.scree_attn_bwd_gqa, (do, q, k, v, o, lse, dq, dk, dv, delta), (do, q, k, v, o, dq, dk, dv))
+    torch.cuda.synchronize()
+    return o, lse, dq, dk, dv
+
+
+@pytest.mark.parametrize("heads", [4, 84])
+@pytest.mark.parametrize("dim", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fp32_scale_of_zero_or_less(dim, heads, causal):
+    """A negative scale is the positive one on -q, and a scale of 0 any scale on
+    q = 0 with no gradient to q and k: the same products in the same order, so
+    the results are equal bit for bit.  (A mask of -inf on the scores would turn
+    into +inf or NaN here.)"""
+    lengths = [1, 33, 70, 129]
+    say(f"case: fp32 scale <= 0, H={heads} D={dim} causal={causal}")
+    _, cu = cu_of(lengths)
+    n, scale = sum(lengths), dim ** -0.5
+    q, do = (randn((n, heads, dim), torch.float32, 60 + i) for i in range(2))
+    k, v = (randn((n, heads // 2, dim), torch.float32, 62 + i) for i in range(2))
+    o, lse, dq, dk, dv = _c_abi_step(-q, k, v, do, cu, causal, scale)
+    for got, want in zip(_c_abi_step(q, k, v, do, cu, causal, -scale), (o, lse, -dq, dk, dv)):
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+    o, lse, _, _, dv = _c_abi_step(torch.zeros_like(q), k, v, do, cu, causal, scale)
+    zero = torch.zeros_like
+    for got, want in zip(_c_abi_step(q, k, v, do, cu, causal, 0.0), (o, lse, zero(q), zero(k), dv)):
+        assert torch.isfinite(want).all() and torch.equal(got, want)
