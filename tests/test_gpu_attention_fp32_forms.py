@@ -98,3 +98,28 @@ def test_fp32_scale_of_zero_or_less(dim, heads, causal):
     zero = torch.zeros_like
     for got, want in zip(_c_abi_step(q, k, v, do, cu, causal, 0.0), (o, lse, zero(q), zero(k), dv)):
         assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("heads", [4, 84])
+@pytest.mark.parametrize("dim", [16, 64, 256])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fp32_scores_keep_every_bit(dim, heads, causal):
+    """Whole-number q and k and a scale that is a power of two: the scores are
+    exact, so adding 512 to 2,048 (by head_dim) to all of them leaves the output
+    as it is, to the rounding of the weights (an ulp of the exponential, and up
+    to 24 * 2^-24 in the exponent of one that counts) and of the sums.  Scores
+    rounded in units of log2(e) would be off by up to 2^-13 there."""
+    lengths = [1, 33, 70, 129]
+    say(f"case: fp32 exact scores, H={heads} D={dim} causal={causal}")
+    _, cu = cu_of(lengths)
+    n, scale = sum(lengths), dim ** -0.5
+    q, k = ((2 * randn((n, heads, dim), torch.float32, 80 + i)).round().clamp(-3, 3) for i in range(2))
+    v, do = (randn((n, heads, dim), torch.float32, 82 + i) for i in range(2))
+    k[..., 0] = 8.0
+    outs = []
+    for shift in (0.0, 1024.0):
+        q[..., 0] = shift
+        outs.append(_c_abi_step(q, k, v, do, cu, causal, scale)[0])
+    worst = float((outs[1] - outs[0]).abs().max())
+    say(f"  largest difference {worst:.2e}")
+    assert worst <= 2.0 ** -20 * float(v.abs().max())
