@@ -2649,9 +2649,45 @@ __global__ __launch_bounds__(kThreads, (D == 64 && KG == 2 ? 3 : f32m_waves<D>()
   if (h == 0 && part == 0 && L > 0) publish_item(src, item, it);
 }
 
+// Delta = rowsum(O * dO) of row r from its row fragments, in the order in which
+// f32m_dot sums dP: the matrix instruction is two FMAs, of half g = 0 and then of
+// g = 1.  A row with few keys has dP close to Delta, and two different orders
+// left their difference as 1.3 times the error of dQ and dK over sequences of 2
+// tokens, 1.16 over 8.  A swap of the two halves of fragments of neighbouring
+// chunks gives lane half g the chunks 2p + g whole.
+template <int D, int FR>
+__device__ __forceinline__ float f32m_delta(const float (&o)[f32m_buf<D>()], const float (&dout)[f32m_buf<D>()]) {
+  constexpr int NC = D / (8 * FR);
+  float delta = 0.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto swap = [](float a, float b, float& half0, float& half1) {
+    const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    half0 = __builtin_bit_cast(float, (unsigned)x[0]);
+    half1 = __builtin_bit_cast(float, (unsigned)x[1]);
+  };
+#pragma unroll
+  for (int c = 0; c < NC; c += 2) {
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 4 * FR * c; i < 4 * FR * (c + 1); ++i) {
+      const bool two = c + 1 < NC;  // (one chunk in all at head_dim 16: lane half 1 sums zeros)
+      float o0, o1, d0, d1;
+      swap(o[i], two ? o[i + 4 * FR] : 0.f, o0, o1);
+      swap(dout[i], two ? dout[i + 4 * FR] : 0.f, d0, d1);
+      acc = fmaf(o1, d1, fmaf(o0, d0, acc));
+    }
+    const float pair = halves_sum(acc);
+    delta = c == 0 ? pair : delta + pair;
+  }
+#else
+  (void)o, (void)dout;
+#endif
+  return delta;
+}
+
 // dQ = scale * dS K with dS = P (dP - Delta), P = exp(S - LSE), dP = dO V^T;
-// Delta = rowsum(O * dO) is formed here and written out for the dK/dV pass.
-// The scores are transposed (keys x queries), as in the forward.
+// Delta is formed here and written out for the dK/dV pass.  The scores are
+// transposed (keys x queries), as in the forward.
 template <int D>
 constexpr bool f32m_op_lds() {  // backward: two row operands per wave
   return D >= 64;
@@ -2695,10 +2731,7 @@ __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dq_f32m_
     t.init(sq.row, r, g);
     t.rows(qv, q + (int64_t)start * sq.row + (int64_t)h * sq.head, qw0, L);
     lse2 = lse[(int64_t)(start + min(qw0 + r, L - 1)) * heads + h] * kLog2e;
-    float d[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < D / 2; ++i) d[i & 3] = fmaf(X[i], dov[i], d[i & 3]);
-    dl = halves_sum((d[0] + d[1]) + (d[2] + d[3]));
+    dl = f32m_delta<D, f32m_chunk<KG>()>(X, dov);
     if (kg == 0 && g == 0 && qw0 + r < L) delta[(int64_t)(start + qw0 + r) * heads + h] = dl;
   }
   float* ql = smem + (wave / KG) * 2 * 32 * SD + r * SD + 4 * g;  // this lane's fragments of Q, then dO
@@ -2762,7 +2795,9 @@ __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dq_f32m_
 // over the query heads that share their K/V head.  The wave's K and V rows
 // are staged in LDS from head_dim 64 up (in registers with the rest they
 // would spill), the waves of a row tile sharing one copy.
-template <int D, bool CAUSAL, int KG>
+// Chunks of FR fragments, as the dQ pass of the same launch takes them (it
+// shares a row tile among no more waves): dP and Delta in one order.
+template <int D, bool CAUSAL, int KG, int FR = f32m_chunk<KG>()>
 __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dkv_f32m_kernel(
     const float* __restrict__ dout, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ lse, const float* __restrict__ delta,
@@ -2859,11 +2894,11 @@ __global__ __launch_bounds__(kThreads, (f32m_waves<D>())) void attn_bwd_dkv_f32m
       }
       if (more) stat = row_stat(hk * group + gi, qb + r);
       __builtin_amdgcn_sched_barrier(0);
-      f32x16 s = f32m_dot<D, f32m_chunk<KG>()>(X, kfrag);
+      f32x16 s = f32m_dot<D, FR>(X, kfrag);
       __builtin_amdgcn_sched_barrier(0);
       to.cols(X, cdh, cur, L);
       __builtin_amdgcn_sched_barrier(0);
-      f32x16 dp = f32m_dot<D, f32m_chunk<KG>()>(Y, vfrag);
+      f32x16 dp = f32m_dot<D, FR>(Y, vfrag);
       __builtin_amdgcn_sched_barrier(0);
       tq.cols(Y, cqh, cur, L);
       __builtin_amdgcn_sched_barrier(0);
@@ -3144,11 +3179,12 @@ template <int KG>
 dim3 f32m_grid(int64_t blocks) {  // whole groups of kXcds * KG (f32m_block)
   return dim3((unsigned)((blocks + kXcds - 1) / kXcds * kXcds * KG));
 }
-// KERNEL for this launch's share, or, at head_dim 256, FMA_KERNEL.  A row
+// KERNEL (KERNEL4: at 4 waves per row tile) for this launch's share, or, at
+// head_dim 256, FMA_KERNEL.  A row
 // tile that sweeps its sequence `sweeps` times (dK/dV: the query heads of a
 // group) has as much the longer a chain: 16 heads on 4 K/V heads of 64, 1,264
 // row tiles, dK/dV 249 us at 4 waves per tile, 417 at 2.
-#define SCREE_LAUNCH_F32(KERNEL, FMA_KERNEL, D, C, blocks, sweeps, stream, ...)                    \
+#define SCREE_LAUNCH_F32(KERNEL, KERNEL4, FMA_KERNEL, D, C, blocks, sweeps, stream, ...)           \
   do {                                                                                             \
     const int64_t blocks_ = (blocks);                                                              \
     if constexpr (D > 128) {                                                                       \
@@ -3157,7 +3193,7 @@ dim3 f32m_grid(int64_t blocks) {  // whole groups of kXcds * KG (f32m_block)
     } else {                                                                                       \
       const int share_ = f32m_share<D>(blocks_ / (sweeps));                                        \
       if (share_ == 4)                                                                             \
-        hipLaunchKernelGGL((KERNEL<D, C, 4>), f32m_grid<4>(blocks_), dim3(kThreads), 0, stream,    \
+        hipLaunchKernelGGL(KERNEL4, f32m_grid<4>(blocks_), dim3(kThreads), 0, stream,              \
                            __VA_ARGS__);                                                           \
       else if (share_ == 2)                                                                        \
         hipLaunchKernelGGL((KERNEL<D, C, 2>), f32m_grid<2>(blocks_), dim3(kThreads), 0, stream,    \
@@ -3173,8 +3209,8 @@ void launch_fwd_f32(const void* q, const void* k, const void* v, void* o, float*
                     const int32_t* cu, int batch, int heads, int kv_heads, const int64_t* st,
                     float scale, int tmax, void* ws, int total, hipStream_t stream) {
   const int hm = attn_head_major(heads, tmax);
-  SCREE_LAUNCH_F32(attn_fwd_f32m_kernel, attn_fwd_f32_kernel, D, C, (int64_t)tmax * heads, 1,
-                   stream, static_cast<const float*>(q), static_cast<const float*>(k),
+  SCREE_LAUNCH_F32(attn_fwd_f32m_kernel, (attn_fwd_f32m_kernel<D, C, 4>), attn_fwd_f32_kernel, D, C,
+                   (int64_t)tmax * heads, 1, stream, static_cast<const float*>(q), static_cast<const float*>(k),
                    static_cast<const float*>(v), static_cast<float*>(o), lse,
                    fwd_item_source(ws, cu, batch, total, tmax, heads, D, hm), tmax, hm, heads,
                    heads / kv_heads, Strides{st[0], st[1]}, Strides{st[2], st[3]},
@@ -3188,8 +3224,8 @@ void launch_bwd_dq_f32(const void* dout, const void* q, const void* k, const voi
                        int kv_heads, const int64_t* st, float scale, int tmax, const void* ws,
                        int total, hipStream_t stream) {
   const int hm = attn_head_major(heads, tmax);
-  SCREE_LAUNCH_F32(attn_bwd_dq_f32m_kernel, attn_bwd_dq_f32_kernel, D, C, (int64_t)tmax * heads,
-                   1, stream, static_cast<const float*>(dout), static_cast<const float*>(q),
+  SCREE_LAUNCH_F32(attn_bwd_dq_f32m_kernel, (attn_bwd_dq_f32m_kernel<D, C, 4>), attn_bwd_dq_f32_kernel, D, C,
+                   (int64_t)tmax * heads, 1, stream, static_cast<const float*>(dout), static_cast<const float*>(q),
                    static_cast<const float*>(k), static_cast<const float*>(v),
                    static_cast<const float*>(o), lse, delta, static_cast<float*>(dq),
                    list_item_source(ws, total, tmax, hm), tmax, hm, heads, heads / kv_heads,
@@ -3205,8 +3241,10 @@ void launch_bwd_dkv_f32(const void* dout, const void* q, const void* k, const vo
                         int kv_heads, const int64_t* st, float scale, int tmax, const void* ws,
                         int total, hipStream_t stream) {
   const int hm = attn_head_major(kv_heads, tmax);
-  SCREE_LAUNCH_F32(attn_bwd_dkv_f32m_kernel, attn_bwd_dkv_f32_kernel, D, C,
-                   (int64_t)tmax * kv_heads, heads / kv_heads, stream, static_cast<const float*>(dout),
+  SCREE_LAUNCH_F32(attn_bwd_dkv_f32m_kernel,
+                   (f32m_share<D>((int64_t)tmax * heads) == 4 ? attn_bwd_dkv_f32m_kernel<D, C, 4>
+                                                              : attn_bwd_dkv_f32m_kernel<D, C, 4, f32m_chunk<2>()>),
+                   attn_bwd_dkv_f32_kernel, D, C, (int64_t)tmax * kv_heads, heads / kv_heads, stream, static_cast<const float*>(dout),
                    static_cast<const float*>(q), static_cast<const float*>(k),
                    static_cast<const float*>(v), lse, delta, static_cast<float*>(dk),
                    static_cast<float*>(dv), list_item_source(ws, total, tmax, hm), tmax, hm,

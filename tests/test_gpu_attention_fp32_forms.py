@@ -123,3 +123,23 @@ def test_fp32_scores_keep_every_bit(dim, heads, causal):
     worst = float((outs[1] - outs[0]).abs().max())
     say(f"  largest difference {worst:.2e}")
     assert worst <= 2.0 ** -20 * float(v.abs().max())
+
+
+@pytest.mark.parametrize("heads", [4, 32])
+@pytest.mark.parametrize("dim", [16, 32, 64, 128, 256])
+def test_fp32_one_key_has_no_score_gradient(dim, heads):
+    """Sequences of one token with a score of 0: the only weight is 1 and the
+    output the value, so dP and Delta are the same products, summed in the same
+    order in both backward passes, and dQ (with q = 0) and dK (with k = 0) are 0.
+    96 sequences, 4 query heads per K/V head: dQ with 4 waves per row tile at 4
+    heads and one at 32, dK/dV with 4."""
+    n = 96
+    say(f"case: fp32 one key, H={heads} D={dim}")
+    _, cu = cu_of([1] * n)
+    q, do = (randn((n, heads, dim), torch.float32, 90 + i) for i in range(2))
+    k, v = (randn((n, heads // 4, dim), torch.float32, 92 + i) for i in range(2))
+    o, _, dq, _, _ = _c_abi_step(torch.zeros_like(q), k, v, do, cu, True, dim ** -0.5)
+    assert torch.equal(o, v.repeat_interleave(4, dim=1))
+    assert not dq.any()
+    _, _, _, dk, _ = _c_abi_step(q, torch.zeros_like(k), v, do, cu, True, dim ** -0.5)
+    assert not dk.any()
