@@ -163,15 +163,11 @@ __device__ __forceinline__ void wave_columns(float (&v)[VEC], int ct, Op op) {
   }
 }
 
-// Merge the partial (max, sum) of other rows into (m, l).  A partial that has
-// seen only -inf and NaN has m = -inf with a NaN sum: l * 0 carries it (0 * 0
-// = 0 otherwise), and two +inf maxima give exp(inf - inf) = NaN.
-__device__ __forceinline__ void sm_merge(float& m, float& l, float m2, float l2) {
-  const float hi = fmaxf(m, m2);
-  const float a = m == -__builtin_inff() ? l * 0.f : l * __builtin_amdgcn_exp2f((m - hi) * kLog2eSm);
-  const float b = m2 == -__builtin_inff() ? l2 * 0.f : l2 * __builtin_amdgcn_exp2f((m2 - hi) * kLog2eSm);
-  l = a + b;
-  m = hi;
+// The sum l of rows with maximum m against a maximum hi >= m of more rows.  A
+// partial that has seen only -inf and NaN has m = -inf with a NaN sum: l * 0
+// carries it (0 * 0 = 0 otherwise), and a +inf maximum gives exp(inf - inf) = NaN.
+__device__ __forceinline__ float sm_rescale(float m, float l, float hi) {
+  return m == -__builtin_inff() ? l * 0.f : l * __builtin_amdgcn_exp2f((m - hi) * kLog2eSm);
 }
 
 // Workgroup -> (sequence, column chunk) index.  Block b runs on XCD b mod 8.
@@ -306,7 +302,11 @@ __global__ __launch_bounds__(kSmThreadsFwd, 6) void varlen_softmax_kernel(
   }
   wave_columns<VEC>(l, ct, [](float a, float b) { return a + b; });
   // The waves' (max, sum) meet in LDS: one thread per column merges them in
-  // wave order (two barriers in all, whatever the number of row lanes).
+  // wave order, every exponential against the columns' maximum and so all at
+  // once (two barriers in all, whatever the number of row lanes).  One wave
+  // after the other, a chain of 14 exponentials, 8,722 rows of 4,819 bf16
+  // columns in 68 sequences took 155 us against 151, 1,026 x 2,934 fp16 in 7
+  // 15.1 against 14.6.
   constexpr int WAVES = kSmThreads / 64;
   const int cols = ct * VEC;
   if ((threadIdx.x & 63) < ct) {
@@ -318,9 +318,17 @@ __global__ __launch_bounds__(kSmThreadsFwd, 6) void varlen_softmax_kernel(
   }
   __syncthreads();
   if ((int)threadIdx.x < cols) {
-    float mm = red_m[threadIdx.x], ll = red_l[threadIdx.x];
+    float mq[WAVES], lq[WAVES];
 #pragma unroll
-    for (int q = 1; q < WAVES; ++q) sm_merge(mm, ll, red_m[q * cols + threadIdx.x], red_l[q * cols + threadIdx.x]);
+    for (int q = 0; q < WAVES; ++q) {
+      mq[q] = red_m[q * cols + threadIdx.x];
+      lq[q] = red_l[q * cols + threadIdx.x];
+    }
+    float mm = mq[0], ll = 0.f;
+#pragma unroll
+    for (int q = 1; q < WAVES; ++q) mm = fmaxf(mm, mq[q]);
+#pragma unroll
+    for (int q = 0; q < WAVES; ++q) ll += sm_rescale(mq[q], lq[q], mm);
     red_m[threadIdx.x] = mm;
     red_l[threadIdx.x] = 1.0f / ll;
   }
