@@ -72,3 +72,31 @@ def test_unaligned_buffers(monkeypatch, dtype, dim):
         _rms_case(dtype, (rows, dim), with_w=True)
         _ln_case(dtype, (rows, dim), params="wb")
         _add_case(dtype, (rows, dim), with_w=True, with_dh=True)
+
+
+@pytest.mark.parametrize("dtype,dim,off", [
+    (torch.float32, 5, 0), (torch.float32, 301, 0), (torch.float32, 768, 1), (torch.float32, 1001, 0),
+    (torch.float32, 2999, 0), (torch.float16, 130, 0), (torch.float16, 770, 0), (torch.float16, 4095, 0)])
+def test_layernorm_xhat_far_from_zero(dtype, dim, off):
+    """The weight gradient sum(dy * x-hat) of rows 1,000 standard deviations from
+    zero, given their statistics: x - 1,000 is a multiple of 1/2 and dy +-1, so
+    x-hat = (x - mean) * rstd has the rounding of two operations, and the sum at
+    most 2^-24 per addition (as many as rows) of the sum of magnitudes.  The
+    rounding of mean * rstd, left in x-hat, is up to 2^-14."""
+    from scree_amd.kernels.hip import norms
+
+    rows = 35
+    g = torch.Generator().manual_seed(dim + rows)
+    x = (1000 + 0.5 * torch.randint(-2, 3, (rows, dim), generator=g)).to(dtype)
+    dy = (2 * torch.randint(0, 2, (rows, dim), generator=g) - 1).to(dtype)
+    x, dy = (torch.cat([torch.zeros(off, dtype=dtype), t.reshape(-1)]).cuda()[off:].view(rows, dim) for t in (x, dy))
+    mean = torch.full((rows,), 1000.0, device="cuda")
+    rstd = (0.5 + 1.5 * torch.rand(rows, generator=g)).cuda()  # mean * rstd is not a float
+    w = torch.ones(dim, dtype=dtype, device="cuda")
+    _, dw, db = norms.layernorm_bwd(dy, x, w, mean, rstd, True, True, p_like=w.float())
+    terms = dy.double() * (x.double() - 1000) * rstd.double()[:, None]
+    bound = (rows + 2) * 2.0 ** -24 * terms.abs().sum(0)
+    err = (dw.double() - terms.sum(0)).abs()
+    print(f"case: LayerNorm x-hat {dtype} {rows} x {dim} + {off}: {float((err / bound).max()):.3f} of the bound", flush=True)
+    assert (err <= bound).all()
+    assert torch.equal(db.double(), dy.double().sum(0))
