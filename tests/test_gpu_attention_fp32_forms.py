@@ -1,30 +1,54 @@
 """GPU parity of the fp32 matrix-instruction attention at the sizes where its
 forms can go wrong: sequence lengths around the 32-row tile and the 128-row
-item, with 4, 2 and 1 waves sharing a row tile (the launchers choose by the
-number of row tiles: 4 below 2,048, or 1,024 from head_dim 64 up; 2 below
-5,120, or 3,072 at head_dim 128), in both mask modes, with and without grouped
+item, with 4, 2 and 1 waves sharing a row tile in each pass (the launchers
+choose by the number of row tiles, for dK/dV as if its launch were the smaller
+by the query heads per K/V head), in both mask modes, with and without grouped
 K/V heads.  Bounds as in ``test_gpu_attention_fp32``.
 """
 
 import pytest
 import torch
 
-from parity import cu_of, randn, say
-from test_gpu_attention_fp32 import run_fp32_case
+from parity import cu_of, np64, randn, say
+from test_gpu_attention_fp32 import TOL, run_fp32_case
 
 pytestmark = pytest.mark.gpu
 
-# 19 row blocks per head (ceil(868 / 128) + 12), 76 row tiles
 TILE_LENGTHS = [1, 31, 32, 33, 64, 65, 96, 127, 128, 129, 160, 2]
+MANY_LENGTHS = TILE_LENGTHS + [(7 * i) % 30 + 1 for i in range(48)]
 
 
-@pytest.mark.parametrize("heads", [8, 32, 84])  # 608, 2,432 and 6,384 row tiles: 4, 2, 1 waves
+def shares(lengths, dim, heads, kv_heads):
+    """Waves per row tile of the forward and dQ, and of dK/dV (the launchers'
+    rule restated, so that each case knows which kernels it runs)."""
+    def share(blocks):
+        tiles = 4 * blocks
+        if tiles < (1024 if dim >= 64 else 2048):
+            return 4
+        return 2 if tiles < (3072 if dim >= 128 else 5120) else 1
+
+    tmax = -(-sum(lengths) // 128) + len(lengths)
+    return share(tmax * heads), share(tmax * kv_heads // (heads // kv_heads))
+
+
+@pytest.mark.parametrize("heads,waves", [(8, 4), (32, 2), (84, 1)])  # 608, 2,432 and 6,384 row tiles
 @pytest.mark.parametrize("dim", [16, 32, 64, 128])
 @pytest.mark.parametrize("causal", [True, False])
-def test_fp32_waves_per_row_tile(dim, heads, causal):
-    # grouped K/V heads below 64 columns; without them the dK/dV pass takes the same form
-    run_fp32_case(TILE_LENGTHS, heads, dim, causal, seed=900 + dim,
-                  kv_heads=heads // 2 if dim < 64 else heads)
+def test_fp32_waves_per_row_tile(dim, heads, waves, causal):
+    assert shares(TILE_LENGTHS, dim, heads, heads) == (waves, waves)
+    run_fp32_case(TILE_LENGTHS, heads, dim, causal, seed=900 + dim)
+
+
+@pytest.mark.parametrize("dim,heads,waves", [
+    (16, 4, (4, 4)), (16, 12, (2, 4)), (16, 32, (1, 2)), (16, 72, (1, 1)),
+    (32, 4, (4, 4)), (32, 12, (2, 4)), (32, 32, (1, 2)), (32, 72, (1, 1)),
+    (64, 2, (4, 4)), (64, 12, (2, 4)), (64, 16, (2, 2)), (64, 72, (1, 1)),
+    (128, 2, (4, 4)), (128, 8, (2, 4)), (128, 16, (1, 2)), (128, 44, (1, 1))])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fp32_waves_per_row_tile_grouped(dim, heads, waves, causal):
+    """Two query heads per K/V head: each dK/dV form steps to the next head of a group."""
+    assert shares(MANY_LENGTHS, dim, heads, heads // 2) == waves
+    run_fp32_case(MANY_LENGTHS, heads, dim, causal, seed=950 + dim, kv_heads=heads // 2)
 
 
 @pytest.mark.parametrize("dim", [16, 64, 128])
@@ -77,7 +101,7 @@ def _c_abi_step(q, k, v, do, cu, causal, scale):
     return o, lse, dq, dk, dv
 
 
-@pytest.mark.parametrize("heads", [4, 84])
+@pytest.mark.parametrize("heads", [4, 84, 216])
 @pytest.mark.parametrize("dim", [16, 32, 64, 128, 256])
 @pytest.mark.parametrize("causal", [True, False])
 def test_fp32_scale_of_zero_or_less(dim, heads, causal):
@@ -100,7 +124,7 @@ def test_fp32_scale_of_zero_or_less(dim, heads, causal):
         assert torch.isfinite(want).all() and torch.equal(got, want)
 
 
-@pytest.mark.parametrize("heads", [4, 84])
+@pytest.mark.parametrize("heads", [4, 84, 216])
 @pytest.mark.parametrize("dim", [16, 64, 256])
 @pytest.mark.parametrize("causal", [True, False])
 def test_fp32_scores_keep_every_bit(dim, heads, causal):
@@ -143,3 +167,48 @@ def test_fp32_one_key_has_no_score_gradient(dim, heads):
     assert not dq.any()
     _, _, _, dk, _ = _c_abi_step(q, torch.zeros_like(k), v, do, cu, True, dim ** -0.5)
     assert not dk.any()
+
+
+def _fwd64(q, k, v, lengths, causal, scale):
+    """Masked softmax attention in fp64 by torch, non-finite scores included."""
+    outs, a = [], 0
+    for n in lengths:
+        qq, kk, vv = (t[a:a + n].double().cpu().transpose(0, 1) for t in (q, k, v))
+        a += n
+        s = qq @ kk.transpose(1, 2) * scale
+        if causal:
+            s = s.masked_fill(~torch.ones(n, n, dtype=torch.bool).tril(), float("-inf"))
+        outs.append((torch.softmax(s, -1) @ vv).transpose(0, 1))
+    return torch.cat(outs).numpy()
+
+
+@pytest.mark.parametrize("heads", [2, 84, 200])  # 4, 2 and 1 waves per row tile
+@pytest.mark.parametrize("dim", [16, 32, 64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fp32_non_finite_scores(dim, heads, causal):
+    """A first tile of keys with scores of -inf (no weight, and NaN for the rows
+    that see nothing else) and a NaN key (NaN for the rows that see it): as in the
+    plain formula, and nothing changes in the other sequences, gradients included."""
+    import numpy as np
+
+    lengths = [70, 129, 33, 90]
+    say(f"case: fp32 non-finite scores, H={heads} D={dim} causal={causal}")
+    _, cu = cu_of(lengths)
+    n, scale = sum(lengths), dim ** -0.5
+    q, k, v, do = (randn((n, heads, dim), torch.float32, 20 + i) for i in range(4))
+    q[..., 0] = 1.0
+    clean = _c_abi_step(q, k, v, do, cu, causal, scale)
+    bad = k.clone()
+    bad[70:102, :, 0] = float("-inf")  # the second sequence's first 32 keys
+    bad[199 + 40] = float("nan")       # past the third: key 7 of the last sequence
+    got = _c_abi_step(q, bad, v, do, cu, causal, scale)
+    want = _fwd64(q, bad, v, lengths, causal, scale)
+    o = np64(got[0])
+    assert np.array_equal(np.isnan(o), np.isnan(want))
+    assert np.nanmax(np.abs(o - want)) <= TOL + 2.0 ** -24 * np.nanmax(np.abs(want))
+    assert np.isnan(want[70:102]).all() if causal else not np.isnan(want[70:199]).any()
+    for a, b in zip(got, clean):
+        assert torch.isfinite(b).all()
+        assert torch.equal(a[:70], b[:70]) and torch.equal(a[199:232], b[199:232])
+    if causal:  # the rows before the NaN key
+        assert torch.equal(got[0][232:239], clean[0][232:239])

@@ -100,3 +100,39 @@ def test_layernorm_xhat_far_from_zero(dtype, dim, off):
     print(f"case: LayerNorm x-hat {dtype} {rows} x {dim} + {off}: {float((err / bound).max()):.3f} of the bound", flush=True)
     assert (err <= bound).all()
     assert torch.equal(db.double(), dy.double().sum(0))
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.float32, 5), (torch.float32, 301), (torch.bfloat16, 128),
+                                       (torch.float16, 770), (torch.bfloat16, 1536), (torch.bfloat16, 4095)])
+def test_non_finite_rows_stay_alone(dtype, dim):
+    """A NaN as a row's last element (repeated by an odd width's last vector) and
+    an infinity as another's first: those rows as the formulas give them, every
+    other row bit for bit as without them, and NaN in the parameter gradients."""
+    from scree_amd.kernels.hip import norms
+
+    print(f"case: non-finite rows {dtype} x {dim}", flush=True)
+    rows, randn = 37, test_gpu_norms.randn
+    x, r, dy = (randn((rows, dim), dtype, 7 + i) for i in range(3))
+    w, b = (randn((dim,), dtype, 10 + i) for i in range(2))
+    bad = x.clone()
+    bad[3, -1], bad[20, 0] = float("nan"), float("inf")
+    others = torch.tensor([i not in (3, 20) for i in range(rows)], device="cuda")
+
+    def steps(x):
+        y, rs = norms.rmsnorm_fwd(x, w, 1e-6, True)
+        yield (y, *norms.rmsnorm_bwd(dy, x, w, rs, True, dw_like=w))
+        y, mu, rs = norms.layernorm_fwd(x, w, b, 1e-5, True)
+        yield (y, *norms.layernorm_bwd(dy, x, w, mu, rs, True, True, p_like=w)[:2])
+        h, y, rs = norms.add_rmsnorm_fwd(x, r, w, 1e-6, True)
+        yield (y, *norms.add_rmsnorm_bwd(dy, r, h, w, rs, True, dw_like=w))
+
+    for i, ((y, dx, dw), (y0, dx0, _)) in enumerate(zip(steps(bad), steps(x))):
+        for a, a0 in ((y, y0), (dx, dx0)):
+            assert torch.isfinite(a0).all()
+            assert torch.equal(a[others], a0[others])
+            assert a[3].isnan().all()
+        assert dw.isnan().all()
+        if i == 1:  # LayerNorm: the mean is infinite
+            assert y[20].isnan().all()
+        else:       # RMSNorm: rstd is 0
+            assert y[20, 0].isnan() and not y[20, 1:].any()

@@ -13,7 +13,7 @@ from test_gpu_softmax import _run
 
 pytestmark = pytest.mark.gpu
 
-# three sequences with rows, so 3 * ceil(columns / lanes) workgroups at a width
+# five sequences, so 5 * ceil(columns / lanes) workgroups at a width (empty ones count)
 LENGTHS = [700, 0, 9000, 1, 0]
 
 
