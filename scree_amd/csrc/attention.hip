@@ -2267,9 +2267,13 @@ __global__ __launch_bounds__((f32_threads<D>())) void attn_bwd_dkv_f32_kernel(
 // (its torch branch, reference/varlen_attention.py:90-113), on
 // v_mfma_f32_32x32x2_f32: fp32 operands, products and sums throughout.  A
 // 32x32 score tile at head_dim 64 is 32 of these (64 cycles each) against
-// ~300 cycles of softmax arithmetic, so the kernels are bound by the matrix
-// cores (154 TFLOP/s measured for a large fp32 GEMM on this GPU); FP32 FMAs
-// with operands from LDS, which they replace, reached 12-30 TFLOP/s.
+// ~300 cycles of softmax arithmetic, so large launches are bound by the matrix
+// cores (154 TFLOP/s measured for a large fp32 GEMM on this GPU).  Small ones
+// are bound by their longest row block's chain of tiles: 16 sequences of mean
+// 256, 8 heads of 64, causal, have one wave per SIMD and keep the matrix cores
+// busy 21-28 % of the cycles.  FP32 FMAs with operands from LDS, which these
+// kernels replace, reached 12 TFLOP/s at that size and 44-66 on two sequences
+// of 4,096.
 //
 // Operand layout.  An instruction takes k = 2: lane (r = l % 32, g = l / 32)
 // supplies A[r][g] and B[g][r], and which k index "g" is, is free as long as
@@ -2296,17 +2300,20 @@ __global__ __launch_bounds__((f32_threads<D>())) void attn_bwd_dkv_f32_kernel(
 // for large ones (f32m_share).
 //
 // Measured (16 sequences of mean 256, 8 heads of 64, causal; the FMA kernels
-// before): forward 115 -> 38 us, dQ 109 -> 49, dK/dV 159 -> 63; two sequences
-// of 4,096: 811 -> 337, 810 -> 483, 1,390 -> 654 us (102-107 TFLOP/s of the
-// executed products).
+// before): forward 115 -> 39 us, dQ 109 -> 51, dK/dV 159 -> 63; two sequences
+// of 4,096: 780 -> 314, 787 -> 464, 1,351 -> 621 us (110-112 TFLOP/s of the
+// executed products).  At head_dim 16 half of each second product is padding:
+// 16 of mean 256 57/59/84 -> 25/28/44 us.
 //
 // Rounding: a dot product over D is summed in chunks of 16 columns (8 columns
 // at KG = 4) and then over the chunks in pairs, and every sum over keys or
 // queries per half tile of 16 rows, then over the halves and the tiles.  The
-// error against 64 bits (2-norm, 28 problems over head_dim 32-128, 256-8,192
-// tokens) is 0.95 / 0.99 / 0.96 / 0.93 of the FMA kernels' (out, dQ, dK, dV;
-// geometric means); with one chain per 32-row tile and 16-column chunks
-// throughout it was 1.02 / 1.01 / 0.98 / 0.96, 3-5 % faster at head_dim 64.
+// error against 64 bits (2-norm, 85 problems: head_dim 16-128, sequences of
+// mean 2 to 4,096, grouped or not, q and k ~ 1 to 4 N(0, 1)) is 0.96 / 0.99 /
+// 0.96 / 0.92 of the FMA kernels' (out, dQ, dK, dV; geometric means; 1.12 /
+// 1.17 / 1.16 / 1.03 at most, on sequences of a few tokens).  One chain per
+// 32-row tile and 16-column chunks throughout had 2-7 % more error and ran 3-5 %
+// faster at head_dim 64.
 __device__ __forceinline__ f32x16 mfma2(float a, float b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
